@@ -188,6 +188,22 @@ int xlbh_run(int lattice, int collision, int store, int compute,
              int nx, int ny, int nz, int64_t plane, double omega, double collision_param, int timestep0, int n_steps,
              void* stream);
 
+/* xlbh_run for a caller that knows what its boundary mask holds: bit k of `known` (1u << XLBH_BC_*)
+ * is set if a cell whose id has kind k may occur (XLBH_BC_NONE: ids with an empty table entry),
+ * XLBH_MASK_SOLID if id 255 may; XLBH_MASK_UNKNOWN if the caller does not know, as xlbh_run does.
+ * Ignored when bc_mask is NULL.  The results are those of xlbh_run, in both buffers and bit for
+ * bit; knowing that no other kinds occur lets the library run several steps in one launch.  A
+ * `known` that leaves out a kind which does occur gives wrong populations there. */
+#define XLBH_MASK_SOLID (1u << 30)
+#define XLBH_MASK_UNKNOWN 0xffffffffu
+int xlbh_run_known(int lattice, int collision, int store, int compute,
+                   void* f_a, void* f_b,
+                   const uint8_t* bc_mask, const uint32_t* missing_bits,
+                   const void* aux, const xlbh_bc_desc* bc_table,
+                   int force_mode, const double* force_uniform, const void* force_field,
+                   int nx, int ny, int nz, int64_t plane, double omega, double collision_param, int timestep0,
+                   int n_steps, uint32_t known, void* stream);
+
 /* n_states steps from f_start, keeping every state: state j (the output of step t0 + j) is
  * written to states + j * xlbh_population_bytes(..., plane) bytes, for j = 0 .. n_states - 1.  The forward pass of a
  * checkpointed reverse sweep (xlbh_adjoint_run without XLBH_ADJ_RECOMPUTE); no counterpart in the

@@ -32,6 +32,7 @@ BC_EXTRAPOLATION_OUTFLOW = 9
 BC_GRADS_APPROXIMATION = 10
 FORCE_NONE, FORCE_UNIFORM, FORCE_FIELD = 0, 1, 2
 ADJ_RECOMPUTE, ADJ_BEGIN, ADJ_END = 1, 2, 4
+MASK_SOLID = 1 << 30
 
 ABI_VERSION = 4
 
@@ -51,6 +52,7 @@ _vp = ctypes.c_void_p
 _i = ctypes.c_int
 _d = ctypes.c_double
 _i64 = ctypes.c_int64
+_u32 = ctypes.c_uint32
 _dp = ctypes.POINTER(ctypes.c_double)
 _bcp = ctypes.POINTER(BcDesc)
 
@@ -62,6 +64,8 @@ SIGNATURES = {
     "xlbh_population_bytes": (_i64, [_i, _i, _i, _i, _i, _i64]),
     "xlbh_step": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _dp, _vp, _i, _i, _i, _i64, _d, _d, _i, _vp]),
     "xlbh_run": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _dp, _vp, _i, _i, _i, _i64, _d, _d, _i, _i, _vp]),
+    "xlbh_run_known": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _dp, _vp, _i, _i, _i, _i64, _d, _d, _i, _i,
+                            _u32, _vp]),
     "xlbh_step_slab": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _dp, _vp, _i, _i, _i, _i64, _d, _d, _i, _i,
                             _i, _vp]),
     "xlbh_stream": (_i, [_i, _i, _vp, _vp, _i, _i, _i, _i64, _vp]),

@@ -1,5 +1,5 @@
 // C entry points of the fused step, the error channel and grid validation.
-#include "step.hpp"
+#include "pair.hpp"
 
 namespace xlbh {
 
@@ -158,10 +158,10 @@ int xlbh_step_slab(int lattice, int collision, int store, int compute, const voi
   return dispatch_step(lattice, c);
 }
 
-int xlbh_run(int lattice, int collision, int store, int compute, void* f_a, void* f_b, const uint8_t* bc_mask,
-             const uint32_t* missing_bits, const void* aux, const xlbh_bc_desc* bc_table, int force_mode,
-             const double* force_uniform, const void* force_field, int nx, int ny, int nz, int64_t plane,
-             double omega, double collision_param, int timestep0, int n_steps, void* stream) {
+int xlbh_run_known(int lattice, int collision, int store, int compute, void* f_a, void* f_b, const uint8_t* bc_mask,
+                   const uint32_t* missing_bits, const void* aux, const xlbh_bc_desc* bc_table, int force_mode,
+                   const double* force_uniform, const void* force_field, int nx, int ny, int nz, int64_t plane,
+                   double omega, double collision_param, int timestep0, int n_steps, uint32_t known, void* stream) {
   (void)timestep0;
   clear_error();
   if (int e = validate_step(lattice, collision, store, compute, f_a, f_b, bc_mask, missing_bits, bc_table,
@@ -172,12 +172,28 @@ int xlbh_run(int lattice, int collision, int store, int compute, void* f_a, void
   if (int e = resolve_plane(lattice, store, nx, ny, nz, plane, P)) return e;
   StepCall c{collision, store, compute, f_a, f_b, bc_mask, missing_bits, aux, bc_table,
              force_mode, force_uniform, force_field, nx, ny, nz, P, omega, collision_param, (hipStream_t)stream};
-  for (int t = 0; t < n_steps; ++t) {
-    c.f_in = (t % 2 == 0) ? f_a : f_b;
-    c.f_out = (t % 2 == 0) ? f_b : f_a;
-    if (int e = dispatch_step(lattice, c)) return e;
+  // Each launch writes the buffer it does not read.  An even number of two-step launches, with
+  // one-step launches for the rest and for the last step, leaves both buffers as n_steps one-step
+  // launches do: the newest state in the buffer n_steps selects, the one before it in the other.
+  PairTiles tiles;
+  int pairs = n_steps > 4 && plan_pair(lattice, c, known, tiles) ? (n_steps - 1) / 4 * 2 : 0;
+  for (int t = 0, launch = 0; t < n_steps; ++launch) {
+    c.f_in = (launch % 2 == 0) ? f_a : f_b;
+    c.f_out = (launch % 2 == 0) ? f_b : f_a;
+    const bool two = launch < pairs;
+    if (int e = two ? launch_pair(lattice, c, tiles) : dispatch_step(lattice, c)) return e;
+    t += two ? 2 : 1;
   }
   return 0;
+}
+
+int xlbh_run(int lattice, int collision, int store, int compute, void* f_a, void* f_b, const uint8_t* bc_mask,
+             const uint32_t* missing_bits, const void* aux, const xlbh_bc_desc* bc_table, int force_mode,
+             const double* force_uniform, const void* force_field, int nx, int ny, int nz, int64_t plane,
+             double omega, double collision_param, int timestep0, int n_steps, void* stream) {
+  return xlbh_run_known(lattice, collision, store, compute, f_a, f_b, bc_mask, missing_bits, aux, bc_table, force_mode,
+                        force_uniform, force_field, nx, ny, nz, plane, omega, collision_param, timestep0, n_steps,
+                        XLBH_MASK_UNKNOWN, stream);
 }
 
 int xlbh_record(int lattice, int collision, int store, int compute, const void* f_start, void* states,

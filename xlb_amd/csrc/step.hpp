@@ -104,9 +104,11 @@ struct PullOffsets {
 // Everything after the pull for one cell with boundary id `id` (!= 255), in place on the
 // post-stream populations f: streaming-step BC, collision (+ force), collision-step BC and the
 // extrapolation-outflow update (nse_stepper.py:360-378).
-template <int LAT, int COLL, int FMT, class C, class O>
+// `fin` reads stored populations other than the pulls: fin.own(l, ...) the cell's own pre-stream
+// population l, fin.at(l, ...) another cell's.
+template <int LAT, int COLL, int FMT, class C, class O, class In>
 __device__ __forceinline__ void cell_update(C* f, int id, O cell, int x, int y, int z, const StepParams& p,
-                                            const PopIn<FMT, C, O>& fin) {
+                                            const In& fin) {
   constexpr LatTables T = make_tables(LAT);
   constexpr int Q = T.q;
   const int nx = p.sw.nx, ny = p.sw.ny, nz = p.sw.nz;
@@ -371,8 +373,8 @@ struct StepCall {
   int x0 = 0, x1 = -1;
 };
 
-template <int LAT, int COLL, int FMT, class C>
-int launch_step_t(const StepCall& c) {
+template <int LAT, int FMT>
+StepParams step_params(const StepCall& c) {
   StepParams p;
   p.f_in = c.f_in;
   p.f_out = c.f_out;
@@ -397,6 +399,12 @@ int launch_step_t(const StepCall& c) {
     p.e_in = reinterpret_cast<const int32_t*>(static_cast<const char*>(c.f_in) + off);
     p.e_out = reinterpret_cast<int32_t*>(static_cast<char*>(c.f_out) + off);
   }
+  return p;
+}
+
+template <int LAT, int COLL, int FMT, class C>
+int launch_step_t(const StepCall& c) {
+  const StepParams p = step_params<LAT, FMT>(c);
   // 32-bit per-lane byte offsets reach every plane of the field from its base
   const bool wide = (uint64_t)Lat<LAT>::Q * p.plane * sizeof(typename Fmt<FMT>::raw) > 0xffffffffull;
   const unsigned lds = sizeof(typename Fmt<FMT>::raw) >= 4 ? kStepLdsCap : 0u;

@@ -9,7 +9,7 @@ and store, writing f_1 and returning (f_0, f_1); the caller swaps, as with the r
 Per-mask device state (derived once and re-derived only when the mask tensors change):
 packed missing bits (N uint32), the 256-entry BC table indexed by boundary id, and the aux side
 table of prescribed values.  ``run`` moves the caller's step/swap loop below the C ABI
-(``xlbh_run``).
+(``xlbh_run_known``).
 """
 
 import ctypes
@@ -81,6 +81,7 @@ class IncompressibleNavierStokesStepper(Stepper):
         self._aux = None
         self._has_bc_cells = True
         self._has_solid = False
+        self._mask_holds = 0
         self._bc_cells = None
         self._mask_ref = None
 
@@ -165,6 +166,11 @@ class IncompressibleNavierStokesStepper(Stepper):
         self._table = self._build_table(bc_mask.device)
         self._has_bc_cells = bool(bc_mask.any().item())
         self._has_solid = self._has_bc_cells and bool((bc_mask == 255).any().item())
+        # what the mask may hold (xlbh_run_known): the kinds of this stepper's boundary conditions,
+        # ids of others (their table entry is empty: kind NONE) and solid cells
+        self._mask_holds = 1 << _lib.BC_NONE | (_lib.MASK_SOLID if self._has_solid else 0)
+        for bc in self.boundary_conditions:
+            self._mask_holds |= 1 << bc.kind
         self._bc_cells = None
         nx, ny, nz = field_extents(bc_mask)
         aux_bcs = [bc for bc in self.boundary_conditions if bc.needs_aux_init]
@@ -414,10 +420,10 @@ class IncompressibleNavierStokesStepper(Stepper):
         ``f_0, f_1 = stepper(...); f_0, f_1 = f_1, f_0`` leaves after ``num_steps`` passes."""
         nx, ny, nz, plane, masks, force_mode, fu_ptr, keep, force_field = self._launch_args(f_0, f_1, bc_mask, missing_mask)
         _lib.check(
-            _lib.lib().xlbh_run(
+            _lib.lib().xlbh_run_known(
                 self.lattice_id, self._collision_id(), self.precision_policy.store_format, self.compute_id,
                 _lib.ptr(f_0), _lib.ptr(f_1), *masks, force_mode, fu_ptr, _lib.ptr(force_field),
-                nx, ny, nz, plane, float(omega), self._collision_param(), int(timestep), int(num_steps),
+                nx, ny, nz, plane, float(omega), self._collision_param(), int(timestep), int(num_steps), self._mask_holds,
                 _lib.stream_of(f_0),
             ),
             "IncompressibleNavierStokesStepper.run",
