@@ -190,11 +190,14 @@ int xlbh_run(int lattice, int collision, int store, int compute,
 
 /* xlbh_run for a caller that knows what its boundary mask holds: bit k of `known` (1u << XLBH_BC_*)
  * is set if a cell whose id has kind k may occur (XLBH_BC_NONE: ids with an empty table entry),
- * XLBH_MASK_SOLID if id 255 may; XLBH_MASK_UNKNOWN if the caller does not know, as xlbh_run does.
+ * XLBH_MASK_SOLID if id 255 may; XLBH_MASK_FAR_OUTFLOW if an extrapolation-outflow cell may have a
+ * missing direction l whose source x - c_l - n is more than one cell away from x along an axis (n the
+ * cell's normal; never at a face of the domain without its edges); XLBH_MASK_UNKNOWN if the caller does not know, as xlbh_run does.
  * Ignored when bc_mask is NULL.  The results are those of xlbh_run, in both buffers and bit for
  * bit; knowing that no other kinds occur lets the library run several steps in one launch.  A
  * `known` that leaves out a kind which does occur gives wrong populations there. */
 #define XLBH_MASK_SOLID (1u << 30)
+#define XLBH_MASK_FAR_OUTFLOW (1u << 29)
 #define XLBH_MASK_UNKNOWN 0xffffffffu
 int xlbh_run_known(int lattice, int collision, int store, int compute,
                    void* f_a, void* f_b,
@@ -214,6 +217,14 @@ int xlbh_record(int lattice, int collision, int store, int compute, const void* 
                 const void* force_field, int nx, int ny, int nz, int64_t plane, double omega, double collision_param,
                 int timestep0,
                 int n_states, void* stream);
+
+/* xlbh_record for a caller that knows what its boundary mask holds (`known` as in
+ * xlbh_run_known). */
+int xlbh_record_known(int lattice, int collision, int store, int compute, const void* f_start, void* states,
+                      const uint8_t* bc_mask, const uint32_t* missing_bits, const void* aux,
+                      const xlbh_bc_desc* bc_table, int force_mode, const double* force_uniform,
+                      const void* force_field, int nx, int ny, int nz, int64_t plane, double omega,
+                      double collision_param, int timestep0, int n_states, uint32_t known, void* stream);
 
 /* ---------------------------------------------------------------------------------------
  * Standalone operators (the reference's per-operator Warp kernels).

@@ -32,7 +32,7 @@ BC_EXTRAPOLATION_OUTFLOW = 9
 BC_GRADS_APPROXIMATION = 10
 FORCE_NONE, FORCE_UNIFORM, FORCE_FIELD = 0, 1, 2
 ADJ_RECOMPUTE, ADJ_BEGIN, ADJ_END = 1, 2, 4
-MASK_SOLID = 1 << 30
+MASK_SOLID, MASK_FAR_OUTFLOW = 1 << 30, 1 << 29
 
 ABI_VERSION = 4
 
@@ -94,6 +94,8 @@ SIGNATURES = {
     "xlbh_adjoint_run": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _dp, _vp, _vp, _i,
                               _i, _i, _i64, _d, _d, _i, _i, _vp, _i, _vp]),
     "xlbh_adjoint_workspace_bytes": (_i64, [_i, _i, _i, _i, _i]),
+    "xlbh_record_known": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _dp, _vp, _i, _i, _i, _i64, _d, _d, _i,
+                               _i, _u32, _vp]),
     "xlbh_record": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _dp, _vp, _i, _i, _i, _i64, _d, _d, _i, _i, _vp]),
 }
 

@@ -1,5 +1,6 @@
 // C entry points of the fused step, the error channel and grid validation.
 #include "pair.hpp"
+#include "steps2d.hpp"
 
 namespace xlbh {
 
@@ -172,9 +173,22 @@ int xlbh_run_known(int lattice, int collision, int store, int compute, void* f_a
   if (int e = resolve_plane(lattice, store, nx, ny, nz, plane, P)) return e;
   StepCall c{collision, store, compute, f_a, f_b, bc_mask, missing_bits, aux, bc_table,
              force_mode, force_uniform, force_field, nx, ny, nz, P, omega, collision_param, (hipStream_t)stream};
-  // Each launch writes the buffer it does not read.  An even number of two-step launches, with
-  // one-step launches for the rest and for the last step, leaves both buffers as n_steps one-step
-  // launches do: the newest state in the buffer n_steps selects, the one before it in the other.
+  // Each launch writes the buffer it does not read.  As many launches as n_steps in parity, the last
+  // of them of one step, leave both buffers as n_steps one-step launches do: the newest state in
+  // the buffer n_steps selects, the one before it in the other.
+  if (n_steps > 2 && steps_2d_apply(lattice, c, known)) {
+    const int per = steps_2d_best(c, n_steps - 1);
+    int launches = 1 + (n_steps - 1 + per - 1) / per;
+    launches += (launches ^ n_steps) & 1;
+    for (int k = 0, t = 0; k < launches; ++k) {
+      c.f_in = (k % 2 == 0) ? f_a : f_b;
+      c.f_out = (k % 2 == 0) ? f_b : f_a;
+      const int left = launches - 1 - k, m = left > 0 ? (n_steps - 1 - t + left - 1) / left : 1;
+      if (int e = m > 1 ? launch_steps_2d(c, m, 0) : dispatch_step(lattice, c)) return e;
+      t += m;
+    }
+    return 0;
+  }
   PairTiles tiles;
   int pairs = n_steps > 4 && plan_pair(lattice, c, known, tiles) ? (n_steps - 1) / 4 * 2 : 0;
   for (int t = 0, launch = 0; t < n_steps; ++launch) {
@@ -196,10 +210,12 @@ int xlbh_run(int lattice, int collision, int store, int compute, void* f_a, void
                         XLBH_MASK_UNKNOWN, stream);
 }
 
-int xlbh_record(int lattice, int collision, int store, int compute, const void* f_start, void* states,
+int xlbh_record_known(int lattice, int collision, int store, int compute, const void* f_start, void* states,
                 const uint8_t* bc_mask, const uint32_t* missing_bits, const void* aux, const xlbh_bc_desc* bc_table,
                 int force_mode, const double* force_uniform, const void* force_field, int nx, int ny, int nz,
-                int64_t plane, double omega, double collision_param, int timestep0, int n_states, void* stream) {
+                int64_t plane, double omega, double collision_param, int timestep0, int n_states,
+                      uint32_t known, void* stream) {
+  (void)timestep0;
   clear_error();
   XLBH_REQUIRE(n_states >= 0, "n_states must be >= 0");
   if (n_states == 0) return 0;
@@ -213,12 +229,25 @@ int xlbh_record(int lattice, int collision, int store, int compute, const void* 
   const size_t field_bytes = (size_t)xlbh_population_bytes(lattice, store, nx, ny, nz, (int64_t)P);
   StepCall c{collision, store, compute, f_start, states, bc_mask, missing_bits, aux, bc_table,
              force_mode, force_uniform, force_field, nx, ny, nz, P, omega, collision_param, (hipStream_t)stream};
-  for (int j = 0; j < n_states; ++j) {
+  const int per = steps_2d_apply(lattice, c, known) ? steps_2d_best(c, n_states) : 1;
+  const int launches = (n_states + per - 1) / per;
+  for (int k = 0, j = 0; k < launches; ++k) {
+    const int m = (n_states - j + launches - k - 1) / (launches - k);
     c.f_in = j == 0 ? f_start : static_cast<const char*>(states) + (size_t)(j - 1) * field_bytes;
     c.f_out = static_cast<char*>(states) + (size_t)j * field_bytes;
-    if (int e = dispatch_step(lattice, c)) return e;
+    if (int e = m > 1 ? launch_steps_2d(c, m, field_bytes) : dispatch_step(lattice, c)) return e;
+    j += m;
   }
   return 0;
+}
+
+int xlbh_record(int lattice, int collision, int store, int compute, const void* f_start, void* states,
+                const uint8_t* bc_mask, const uint32_t* missing_bits, const void* aux, const xlbh_bc_desc* bc_table,
+                int force_mode, const double* force_uniform, const void* force_field, int nx, int ny, int nz,
+                int64_t plane, double omega, double collision_param, int timestep0, int n_states, void* stream) {
+  return xlbh_record_known(lattice, collision, store, compute, f_start, states, bc_mask, missing_bits, aux, bc_table,
+                           force_mode, force_uniform, force_field, nx, ny, nz, plane, omega, collision_param, timestep0,
+                           n_states, XLBH_MASK_UNKNOWN, stream);
 }
 
 }  // extern "C"

@@ -259,7 +259,10 @@ __device__ __forceinline__ void collide(C* f, C omega, bool has_force, const C* 
       if (cs >= 2) strain += C(2) * fneq * fneq;
     }
     const C tau0 = C(1) / omega;
-    const C tau = tau0 + C(0.5) * (sqrt(tau0 * tau0 + C(36) * (cparam * cparam) * sqrt(strain)) - tau0);
+    // the fused multiply-add is written out: left to the compiler it covers one product or the other,
+    // depending on whether the kernel has a loop to hoist tau0 * tau0 from
+    const C rad = __builtin_elementwise_fma(tau0, tau0, C(36) * (cparam * cparam) * sqrt(strain));
+    const C tau = tau0 + C(0.5) * (sqrt(rad) - tau0);
     const C inv_tau = C(1) / tau;
 #pragma unroll
     for (int l = 0; l < Q; ++l) {

@@ -171,6 +171,8 @@ class IncompressibleNavierStokesStepper(Stepper):
         self._mask_holds = 1 << _lib.BC_NONE | (_lib.MASK_SOLID if self._has_solid else 0)
         for bc in self.boundary_conditions:
             self._mask_holds |= 1 << bc.kind
+            if self._has_bc_cells and bc.kind == _lib.BC_EXTRAPOLATION_OUTFLOW and self._far_outflow(bc.id, bc_mask):
+                self._mask_holds |= _lib.MASK_FAR_OUTFLOW
         self._bc_cells = None
         nx, ny, nz = field_extents(bc_mask)
         aux_bcs = [bc for bc in self.boundary_conditions if bc.needs_aux_init]
@@ -181,6 +183,19 @@ class IncompressibleNavierStokesStepper(Stepper):
                 bc.aux_data_init(None, None, bc_mask, missing_mask, aux=self._aux)
         self._mask_ref = bc_mask
         self._state_key = self._mask_key(bc_mask, missing_mask)
+
+    def _far_outflow(self, bc_id, bc_mask):
+        """True if a cell of the extrapolation outflow ``bc_id`` reads a source x - c_l - n more than
+        one cell away along an axis (its normal n and its missing directions l taken as the step
+        kernel does, helper_functions_bc.py:75-86)."""
+        c = np.asarray(self.velocity_set.c)
+        main = [l for l in range(self.velocity_set.q) if np.abs(c[:, l]).sum() == 1]
+        for bits in torch.unique(self._bits[bc_mask.view(-1) == int(bc_id)]).tolist():
+            missing = [l for l in range(self.velocity_set.q) if bits >> l & 1]
+            normal = next((-c[:, l] for l in main if l in missing), np.zeros(len(c), dtype=c.dtype))
+            if any(np.abs(c[:, l] + normal).max() > 1 for l in missing):
+                return True
+        return False
 
     def _force_args(self):
         col = self.collision
@@ -311,7 +326,7 @@ class IncompressibleNavierStokesStepper(Stepper):
         return lam_in
 
     def record(self, f_start, states, bc_mask, missing_mask, omega, num_states, timestep=0):
-        """``num_states`` steps from ``f_start`` keeping every state (xlbh_record): states[j] is the
+        """``num_states`` steps from ``f_start`` keeping every state (xlbh_record_known): states[j] is the
         output of step ``timestep + j``.  ``states`` is a contiguous (>= num_states, q, ...) tensor
         in the store dtype."""
         nx, ny, nz, plane, masks, force_mode, fu_ptr, keep, force_field = self._launch_args(f_start, None, bc_mask, missing_mask)
@@ -320,10 +335,10 @@ class IncompressibleNavierStokesStepper(Stepper):
         if num_states > 0:
             self._expect_states(states, num_states, f_start, plane)
         _lib.check(
-            _lib.lib().xlbh_record(
+            _lib.lib().xlbh_record_known(
                 self.lattice_id, self._collision_id(), self.precision_policy.store_format, self.compute_id,
                 _lib.ptr(f_start), _lib.ptr(states), *masks, force_mode, fu_ptr, _lib.ptr(force_field),
-                nx, ny, nz, plane, float(omega), self._collision_param(), int(timestep), int(num_states),
+                nx, ny, nz, plane, float(omega), self._collision_param(), int(timestep), int(num_states), self._mask_holds,
                 _lib.stream_of(f_start),
             ),
             "IncompressibleNavierStokesStepper.record",
