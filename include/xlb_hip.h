@@ -420,6 +420,19 @@ int xlbh_adjoint_run(int lattice, int collision, int store, int compute,
 #define XLBH_ADJ_BEGIN 2
 #define XLBH_ADJ_END 4
 
+/* xlbh_adjoint_run for a caller that knows what its boundary mask holds (`known` as in
+ * xlbh_run_known).  XLBH_MASK_SOLID set makes it check the mask as xlbh_adjoint_run does; without it
+ * the mask is not read for the check and the call does not synchronise. */
+int xlbh_adjoint_run_known(int lattice, int collision, int store, int compute,
+                           const void* f_ckpt, void* states, void* lam_a, void* lam_b,
+                           const uint8_t* bc_mask, const uint32_t* missing_bits,
+                           const void* aux, const xlbh_bc_desc* bc_table,
+                           const int32_t* bc_cells, int n_bc_cells,
+                           int force_mode, const double* force_uniform, const void* force_field,
+                           double* grad_force, int nx, int ny, int nz, int64_t plane, double omega,
+                           double collision_param, int timestep0, int n_steps, void* workspace, int flags,
+                           uint32_t known, void* stream);
+
 /* Bytes of the fused reverse sweep's workspace: three (Q, N) fields of the compute type and N
  * flag bytes, rounded up to 256 (-1 for invalid arguments). */
 int64_t xlbh_adjoint_workspace_bytes(int lattice, int compute, int nx, int ny, int nz);

@@ -6,6 +6,7 @@ loaded (both carry the soname libamdhip64.so.7) and shares its streams and alloc
 """
 
 import ctypes
+import functools
 import os
 
 import torch
@@ -93,6 +94,8 @@ SIGNATURES = {
                                _i, _i64, _d, _d, _vp]),
     "xlbh_adjoint_run": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _dp, _vp, _vp, _i,
                               _i, _i, _i64, _d, _d, _i, _i, _vp, _i, _vp]),
+    "xlbh_adjoint_run_known": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _dp, _vp, _vp,
+                                    _i, _i, _i, _i64, _d, _d, _i, _i, _vp, _i, _u32, _vp]),
     "xlbh_adjoint_workspace_bytes": (_i64, [_i, _i, _i, _i, _i]),
     "xlbh_record_known": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _dp, _vp, _i, _i, _i, _i64, _d, _d, _i,
                                _i, _u32, _vp]),
@@ -131,10 +134,8 @@ def check(rc, what="libxlbhip"):
 
 
 def ptr(t):
-    """Device pointer of a tensor (None -> NULL)."""
-    if t is None:
-        return None
-    return ctypes.c_void_p(t.data_ptr())
+    """Device pointer of a tensor (None -> NULL), as ctypes takes it for a void*."""
+    return None if t is None else t.data_ptr()
 
 
 def require_cuda(*tensors):
@@ -145,8 +146,8 @@ def require_cuda(*tensors):
 
 def stream_of(t=None):
     """hipStream_t (as void*) of torch's current stream on the tensor's device."""
-    dev = t.device if t is not None else torch.device("cuda", torch.cuda.current_device())
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    index = t.device.index if t is not None else None
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def doubles(values):
@@ -154,9 +155,18 @@ def doubles(values):
     return ctypes.cast(arr, _dp), arr
 
 
+_increment_version = getattr(torch.autograd.graph, "increment_version", None)
+
+
 def mark_written(*tensors):
     """Bump torch's version counter of tensors written through raw pointers."""
-    bump = getattr(torch.autograd.graph, "increment_version", None)
-    for t in tensors:
-        if t is not None and bump is not None:
-            bump(t)
+    if _increment_version is not None:
+        for t in tensors:
+            if t is not None:
+                _increment_version(t)
+
+
+@functools.lru_cache(maxsize=256)
+def population_bytes(lattice, store, nx, ny, nz, plane):
+    """xlbh_population_bytes, a function of its arguments alone."""
+    return int(lib().xlbh_population_bytes(lattice, store, nx, ny, nz, plane))

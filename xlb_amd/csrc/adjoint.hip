@@ -120,13 +120,13 @@ static AdjParams adjoint_params(int collision, double cparam, const void* f_in, 
   return p;
 }
 
-extern "C" int xlbh_adjoint_run(int lattice, int collision, int store, int compute, const void* f_ckpt, void* states,
+extern "C" int xlbh_adjoint_run_known(int lattice, int collision, int store, int compute, const void* f_ckpt, void* states,
                                 void* lam_a, void* lam_b, const uint8_t* bc_mask, const uint32_t* missing_bits,
                                 const void* aux, const xlbh_bc_desc* bc_table, const int32_t* bc_cells,
                                 int n_bc_cells, int force_mode, const double* force_uniform,
                                 const void* force_field, double* grad_force, int nx, int ny, int nz, int64_t plane,
                                 double omega, double collision_param, int timestep0, int n_steps, void* workspace,
-                                int flags, void* stream) {
+                                int flags, uint32_t known, void* stream) {
   clear_error();
   if (int e = adjoint_validate(lattice, collision, force_mode, force_uniform, force_field, bc_mask, missing_bits,
                                bc_table, nx, ny, nz))
@@ -141,8 +141,8 @@ extern "C" int xlbh_adjoint_run(int lattice, int collision, int store, int compu
   XLBH_REQUIRE(n_steps == 1 || states, "adjoint_run needs a state workspace for n_steps > 1");
   XLBH_REQUIRE(valid_store(store), "unknown store format");
   // the mask scan synchronises the stream: once per sweep (XLBH_ADJ_BEGIN) with a workspace,
-  // every call without one
-  if (!workspace || (flags & XLBH_ADJ_BEGIN))
+  // every call without one; a caller that knows there is no solid cell is spared it
+  if ((known & XLBH_MASK_SOLID) && (!workspace || (flags & XLBH_ADJ_BEGIN)))
     if (int e = refuse_solid_cells(bc_mask, nx, ny, nz, (hipStream_t)stream)) return e;
   const size_t field_bytes = (size_t)lattice_q(lattice) * P * store_bytes(store);
   auto state = [&](int j) -> const void* {
@@ -197,6 +197,19 @@ extern "C" int xlbh_adjoint_run(int lattice, int collision, int store, int compu
     if (int e = adjoint_dispatch(lattice, store, compute, p, s, ADJ_FLUSH, 0, nullptr, cur)) return e;
   }
   return 0;
+}
+
+extern "C" int xlbh_adjoint_run(int lattice, int collision, int store, int compute, const void* f_ckpt, void* states,
+                                void* lam_a, void* lam_b, const uint8_t* bc_mask, const uint32_t* missing_bits,
+                                const void* aux, const xlbh_bc_desc* bc_table, const int32_t* bc_cells,
+                                int n_bc_cells, int force_mode, const double* force_uniform,
+                                const void* force_field, double* grad_force, int nx, int ny, int nz, int64_t plane,
+                                double omega, double collision_param, int timestep0, int n_steps, void* workspace,
+                                int flags, void* stream) {
+  return xlbh_adjoint_run_known(lattice, collision, store, compute, f_ckpt, states, lam_a, lam_b, bc_mask, missing_bits,
+                                aux, bc_table, bc_cells, n_bc_cells, force_mode, force_uniform, force_field, grad_force,
+                                nx, ny, nz, plane, omega, collision_param, timestep0, n_steps, workspace, flags,
+                                XLBH_MASK_UNKNOWN, stream);
 }
 
 extern "C" int64_t xlbh_adjoint_workspace_bytes(int lattice, int compute, int nx, int ny, int nz) {

@@ -3,7 +3,9 @@
 ``register_backend`` / ``__call__`` keep the reference's dispatch: every implementation
 registered for (class name, backend) is tried with the call's arguments; if none binds and runs,
 a generic ``Exception`` carrying the last error and its traceback is raised
-(operator.py:54-74).  Signatures are computed once at registration instead of on every call.
+(operator.py:54-74).  Signatures are computed once at registration, the implementations of a class
+are looked up once, and a call is bound to a signature only to report why it failed (a call that
+does not bind raises TypeError before the implementation runs).
 """
 
 import inspect
@@ -18,6 +20,7 @@ from xlb_amd.precision_policy import Precision
 class Operator:
     _backends = {}
     _signatures = {}
+    _candidates = {}  # (class, backend) of past calls -> its implementations; cleared by a registration
 
     def __init__(self, velocity_set=None, precision_policy=None, compute_backend=None):
         self.velocity_set = velocity_set or DefaultConfig.velocity_set
@@ -36,30 +39,40 @@ class Operator:
             key = (subclass_name, backend_name, str(signature))
             cls._backends[key] = func
             cls._signatures[key] = signature
+            Operator._candidates.clear()
             return func
 
         return decorator
 
+    def _implementations(self):
+        """[(key, method)] of the first class in the MRO with implementations for the backend."""
+        cached = self._candidates.get((type(self), self.compute_backend.name))
+        if cached is not None:
+            return cached
+        found = []
+        for klass in type(self).__mro__:
+            found = [(k, m) for k, m in self._backends.items() if k[0] == klass.__name__ and k[1] == self.compute_backend]
+            if found:
+                break
+        self._candidates[type(self), self.compute_backend.name] = found
+        return found
+
     def __call__(self, *args, callback=None, **kwargs):
         error, traceback_str, key = None, "", None
-        for klass in type(self).__mro__:
-            candidates = [
-                (k, m) for k, m in self._backends.items() if k[0] == klass.__name__ and k[1] == self.compute_backend
-            ]
-            for key, backend_method in candidates:
-                try:
-                    self._signatures[key].bind(self, *args, **kwargs)
-                    result = backend_method(self, *args, **kwargs)
-                    callback_arg = result if result is not None else (args, kwargs)
-                    if callback and callable(callback):
-                        callback(callback_arg)
-                    return result
-                except Exception as e:  # same contract as the reference: try the next candidate
-                    error = e
-                    traceback_str = traceback.format_exc()
-                    continue
-            if candidates:
-                break
+        for key, backend_method in self._implementations():
+            try:
+                result = backend_method(self, *args, **kwargs)
+                if callback and callable(callback):
+                    callback(result if result is not None else (args, kwargs))
+                return result
+            except Exception as e:  # same contract as the reference: try the next candidate
+                error = e
+                traceback_str = traceback.format_exc()
+            try:
+                self._signatures[key].bind(self, *args, **kwargs)
+            except Exception as e:
+                error = e
+                traceback_str = traceback.format_exc()
         raise Exception(f"Error captured for backend with key {key} for operator {self.__class__.__name__}: {error}\n {traceback_str}")
 
     @property
@@ -108,16 +121,14 @@ def plane_stride(f):
     (``create_field(..., padded=True)``).  None if the field has another layout."""
     if f.dim() != 4:
         return None
-    card, nx, ny, nz = (int(v) for v in f.shape)
+    card, nx, ny, nz = f.shape
+    s = f.stride()
+    if (nz > 1 and s[3] != 1) or (ny > 1 and s[2] != nz) or (nx > 1 and s[1] != ny * nz):
+        return None
     n = nx * ny * nz
-    want = (None, ny * nz, nz, 1)
-    for d in (1, 2, 3):
-        if f.shape[d] > 1 and f.stride(d) != want[d]:
-            return None
     if card == 1:
         return n
-    p = int(f.stride(0))
-    return p if p >= n else None
+    return s[0] if s[0] >= n else None
 
 
 def field_extents(f):
@@ -126,7 +137,7 @@ def field_extents(f):
         raise ValueError(f"fields must have shape (cardinality, nx, ny, nz); got {tuple(f.shape)}")
     if plane_stride(f) is None:
         raise ValueError("fields must be C-ordered (z unit-stride) within each plane")
-    return int(f.shape[1]), int(f.shape[2]), int(f.shape[3])
+    return tuple(f.shape[1:])
 
 
 def expect_population(t, q, extents, name, dtype, lattice, store):
@@ -137,14 +148,14 @@ def expect_population(t, q, extents, name, dtype, lattice, store):
         raise ValueError(f"{name} is required")
     if not t.is_cuda:
         raise ValueError(f"{name} must live on the GPU (device='cuda')")
-    if tuple(t.shape) != (int(q),) + tuple(extents):
+    if t.shape != (int(q),) + tuple(extents):
         raise ValueError(f"{name} has shape {tuple(t.shape)}; expected {(int(q),) + tuple(extents)}")
     if t.dtype != dtype:
         raise ValueError(f"{name} has dtype {t.dtype}; expected {dtype}")
     plane = plane_stride(t)
     if plane is None:
         raise ValueError(f"{name} must be C-ordered within each plane (a contiguous tensor or a plane-padded field)")
-    need = int(_lib.lib().xlbh_population_bytes(lattice, store, *extents, plane))
+    need = _lib.population_bytes(lattice, store, *extents, plane)
     have = t.untyped_storage().nbytes() - t.storage_offset() * t.element_size()
     if need < 0 or have < need:
         what = " and its segment exponents" if store == _lib.I16_BLOCK else ""
@@ -179,7 +190,7 @@ def expect_field(t, cardinality, extents, name, dtype=None):
         raise ValueError(f"{name} is required")
     if not t.is_cuda:
         raise ValueError(f"{name} must live on the GPU (device='cuda')")
-    if tuple(t.shape) != (int(cardinality),) + tuple(extents):
+    if t.shape != (int(cardinality),) + tuple(extents):
         raise ValueError(f"{name} has shape {tuple(t.shape)}; expected {(int(cardinality),) + tuple(extents)}")
     if not t.is_contiguous():
         raise ValueError(f"{name} must be contiguous")

@@ -209,8 +209,10 @@ class IncompressibleNavierStokesStepper(Stepper):
             return _lib.FORCE_UNIFORM, col.force_vector, None
         return _lib.FORCE_NONE, None, None
 
+    _COLLISION_IDS = {"KBC": _lib.KBC, "SmagorinskyLESBGK": _lib.SMAGORINSKY_BGK}
+
     def _collision_id(self):
-        return {"KBC": _lib.KBC, "SmagorinskyLESBGK": _lib.SMAGORINSKY_BGK}.get(self.collision_type, _lib.BGK)
+        return self._COLLISION_IDS.get(self.collision_type, _lib.BGK)
 
     def _collision_param(self):
         return float(getattr(self.collision, "collision_param", 0.0))
@@ -230,7 +232,7 @@ class IncompressibleNavierStokesStepper(Stepper):
         force_mode, force_vec, force_field = self._force_args()
         if force_field is not None:
             expect_field(force_field, self.velocity_set.d, ext, "force_field", self.compute_dtype)
-        fu_ptr, keep = _lib.doubles(force_vec if force_vec is not None else (0.0, 0.0, 0.0))
+        fu_ptr, keep = _lib.doubles(force_vec) if force_vec is not None else (None, None)
         if self._has_bc_cells:
             masks = (_lib.ptr(bc_mask), _lib.ptr(self._bits), _lib.ptr(self._aux), _lib.ptr(self._table))
         else:
@@ -356,8 +358,7 @@ class IncompressibleNavierStokesStepper(Stepper):
         plane = plane_stride(f_like)
         if plane is None:
             raise ValueError("f_like must be C-ordered within each plane")
-        per = int(_lib.lib().xlbh_population_bytes(self.lattice_id, self.precision_policy.store_format, nx, ny, nz,
-                                                   plane))
+        per = _lib.population_bytes(self.lattice_id, self.precision_policy.store_format, nx, ny, nz, plane)
         elem = f_like.element_size()
         if per < 0 or per % elem or (per // elem) % q:
             raise ValueError("state buffers are not available for this store format")
@@ -367,8 +368,7 @@ class IncompressibleNavierStokesStepper(Stepper):
     def _expect_states(self, states, n, f_like, plane):
         q = self.velocity_set.q
         nx, ny, nz = (int(v) for v in f_like.shape[1:])
-        per = int(_lib.lib().xlbh_population_bytes(self.lattice_id, self.precision_policy.store_format, nx, ny, nz,
-                                                   plane))
+        per = _lib.population_bytes(self.lattice_id, self.precision_policy.store_format, nx, ny, nz, plane)
         elem = f_like.element_size()
         want = (per // elem, plane, ny * nz, nz, 1)
         ok = (states is not None and states.dtype == self.store_dtype and states.dim() == 5 and states.shape[0] >= n
@@ -387,7 +387,7 @@ class IncompressibleNavierStokesStepper(Stepper):
 
     def adjoint_run(self, f_ckpt, states, lam_a, lam_b, bc_mask, missing_mask, omega, num_steps, timestep=0,
                     grad_force=None, recompute=True, workspace=None, begin=True, end=True):
-        """Reverse sweep over one checkpoint segment below the ABI (xlbh_adjoint_run): recompute the
+        """Reverse sweep over one checkpoint segment below the ABI (xlbh_adjoint_run_known): recompute the
         ``num_steps - 1`` states after ``f_ckpt`` into ``states`` ((num_steps - 1, q, ...) in the
         store dtype), then apply the adjoint steps in reverse starting from lam_a = dL/df at the
         segment end.  Returns the buffer (lam_a or lam_b) that holds dL/df_ckpt.  With
@@ -417,11 +417,11 @@ class IncompressibleNavierStokesStepper(Stepper):
                 raise ValueError(f"workspace must be a contiguous uint8 tensor of >= {need} bytes")
             flags |= (_lib.ADJ_BEGIN if begin else 0) | (_lib.ADJ_END if end else 0)
         _lib.check(
-            _lib.lib().xlbh_adjoint_run(
+            _lib.lib().xlbh_adjoint_run_known(
                 self.lattice_id, self._collision_id(), self.precision_policy.store_format, self.compute_id,
                 _lib.ptr(f_ckpt), _lib.ptr(states), _lib.ptr(lam_a), _lib.ptr(lam_b), *masks, *self._adjoint_cells(),
                 force_mode, fu_ptr, _lib.ptr(force_field), _lib.ptr(grad_force), nx, ny, nz, plane, float(omega),
-                self._collision_param(), int(timestep), int(num_steps), _lib.ptr(workspace), flags,
+                self._collision_param(), int(timestep), int(num_steps), _lib.ptr(workspace), flags, self._mask_holds,
                 _lib.stream_of(f_ckpt),
             ),
             "IncompressibleNavierStokesStepper.adjoint_run",

@@ -36,15 +36,7 @@ class Precision(Enum):
 
     @property
     def torch_dtype(self):
-        return {
-            Precision.FP64: torch.float64,
-            Precision.FP32: torch.float32,
-            Precision.FP16: torch.float16,
-            Precision.UINT8: torch.uint8,
-            Precision.BOOL: torch.bool,
-            Precision.BF16: torch.bfloat16,
-            Precision.INT16: torch.int16,
-        }[self]
+        return self._torch_dtype
 
     @property
     def field_id(self):
@@ -62,6 +54,20 @@ class Precision(Enum):
         raise ValueError(f"unsupported dtype {dtype}")
 
 
+# The properties below are read several times in every operator call, so each member holds its
+# values instead of looking itself up in a table on every access.
+for _p, _dtype in {
+    Precision.FP64: torch.float64,
+    Precision.FP32: torch.float32,
+    Precision.FP16: torch.float16,
+    Precision.UINT8: torch.uint8,
+    Precision.BOOL: torch.bool,
+    Precision.BF16: torch.bfloat16,
+    Precision.INT16: torch.int16,
+}.items():
+    _p._torch_dtype = _dtype
+
+
 class PrecisionPolicy(Enum):
     FP64FP64 = auto()
     FP64FP32 = auto()
@@ -76,24 +82,11 @@ class PrecisionPolicy(Enum):
 
     @property
     def compute_precision(self):
-        if self in (PrecisionPolicy.FP64FP64, PrecisionPolicy.FP64FP32, PrecisionPolicy.FP64FP16):
-            return Precision.FP64
-        return Precision.FP32
+        return self._compute_precision
 
     @property
     def store_precision(self):
-        return {
-            PrecisionPolicy.FP64FP64: Precision.FP64,
-            PrecisionPolicy.FP64FP32: Precision.FP32,
-            PrecisionPolicy.FP64FP16: Precision.FP16,
-            PrecisionPolicy.FP32FP32: Precision.FP32,
-            PrecisionPolicy.FP32FP16: Precision.FP16,
-            PrecisionPolicy.FP32BF16: Precision.BF16,
-            PrecisionPolicy.FP32FP16_SHIFTED: Precision.FP16,
-            PrecisionPolicy.FP32BF16_SHIFTED: Precision.BF16,
-            PrecisionPolicy.FP32I16_BLOCK: Precision.INT16,
-            PrecisionPolicy.FP32FP32_DEVIATION: Precision.FP32,
-        }[self]
+        return self._store_precision
 
     @property
     def shifted(self):
@@ -108,17 +101,29 @@ class PrecisionPolicy(Enum):
     @property
     def store_format(self):
         """Population storage format id in the C ABI (XLBH_F32 ... XLBH_I16_BLOCK)."""
-        if self.block:
-            return 6
-        base = {Precision.FP32: 0, Precision.FP64: 1, Precision.FP16: 2, Precision.BF16: 3}[self.store_precision]
-        if self.shifted:
-            base += 2
-        return base
+        return self._store_format
 
     @property
     def compute_id(self):
         """Compute type id in the C ABI (XLBH_COMPUTE_F32 / XLBH_COMPUTE_F64 /
         XLBH_COMPUTE_F32_DEVIATION)."""
-        if self == PrecisionPolicy.FP32FP32_DEVIATION:
-            return 2
-        return 1 if self.compute_precision == Precision.FP64 else 0
+        return self._compute_id
+
+
+for _p, _store in {
+    PrecisionPolicy.FP64FP64: Precision.FP64,
+    PrecisionPolicy.FP64FP32: Precision.FP32,
+    PrecisionPolicy.FP64FP16: Precision.FP16,
+    PrecisionPolicy.FP32FP32: Precision.FP32,
+    PrecisionPolicy.FP32FP16: Precision.FP16,
+    PrecisionPolicy.FP32BF16: Precision.BF16,
+    PrecisionPolicy.FP32FP16_SHIFTED: Precision.FP16,
+    PrecisionPolicy.FP32BF16_SHIFTED: Precision.BF16,
+    PrecisionPolicy.FP32I16_BLOCK: Precision.INT16,
+    PrecisionPolicy.FP32FP32_DEVIATION: Precision.FP32,
+}.items():
+    _p._store_precision = _store
+    _p._compute_precision = Precision.FP64 if _p.name.startswith("FP64") else Precision.FP32
+    _p._compute_id = 2 if _p == PrecisionPolicy.FP32FP32_DEVIATION else int(_p._compute_precision == Precision.FP64)
+    _p._store_format = 6 if _p.block else (
+        {Precision.FP32: 0, Precision.FP64: 1, Precision.FP16: 2, Precision.BF16: 3}[_store] + (2 if _p.shifted else 0))
