@@ -730,13 +730,49 @@ __global__ __launch_bounds__(256) void k_adjoint_bc_list(AdjParams p) {
 // neighbour part lands on cell x - c_l - n; it goes to d_nb (double-buffered by step parity) and
 // is read and cleared by the flagged consumer cell in the next reverse step.
 // ------------------------------------------------------------------------------------------
+// Coordinates v + s c for c in {-1, 0, 1} with periodic wrap.
+struct AxisShift {
+  int lo, mid, hi;
+  __device__ __forceinline__ AxisShift(int v, int n, int s) : lo(wrap1(v - s, n)), mid(v), hi(wrap1(v + s, n)) {}
+  __device__ __forceinline__ int operator[](int c) const { return c < 0 ? lo : (c > 0 ? hi : mid); }
+};
+
+// Element (x, y, z) of the plane that starts at element `plane` of a field.  The slow coordinates (x
+// and y in 3-D, x in 2-D) are wave-uniform, so everything but the position along the row is scalar
+// (the empty asm keeps the two parts apart: the scalar-base form of loads and stores).
+template <int LAT, class R>
+__device__ __forceinline__ const R* row_at(const R* base, uint64_t plane, int ny, int nz, int x, int y, int z) {
+  constexpr bool three = make_tables(LAT).d == 3;
+  using gchar = const __attribute__((address_space(1))) char;
+  const uint64_t row = three ? ((uint64_t)x * ny + y) * nz : (uint64_t)x * ny;
+  gchar* b = (gchar*)(base + plane + row);
+  uint32_t o = (uint32_t)(three ? z : y) * (uint32_t)sizeof(R);
+  asm("" : "+s"(b), "+v"(o));
+  return reinterpret_cast<const R*>((const char*)b + o);
+}
+
 __device__ __forceinline__ bool own_kind(int kind) {
   return kind == XLBH_BC_HALFWAY_BB || kind == XLBH_BC_EXTRAPOLATION_OUTFLOW || kind == XLBH_BC_DO_NOTHING ||
          kind == XLBH_BC_GRADS_APPROXIMATION;
 }
 
-template <int LAT, int FMT, class C, int COLL>
-__global__ __launch_bounds__(256) void k_adjoint_fused(AdjParams p) {
+struct SweepForm {
+  int pulled_in, own_out;
+};
+__device__ __forceinline__ SweepForm sweep_form() { return {0, 0}; }
+__device__ __forceinline__ SweepForm sweep_form(SweepForm f) { return f; }
+
+// Between the steps of one sweep dL/df need not be pushed at all: with `own_out` the cell stores its
+// G_ps at its own slots, and with `pulled_in` it reads lam_out,k(x) = G_ps,k(x + c_k) from there.  The
+// reverse step is then shifted loads and aligned stores, as the forward step is (the push, aligned
+// loads and shifted stores, streams 10 % slower), and the stores are non-temporal (for rows of whole
+// 128-byte lines).  SWEEP selects this form; without it the cell
+// reads plain dL/df and pushes (the first and last step of a sweep read and write plain fields in
+// either form).  BCS: the mask may hold boundary cells.
+template <int LAT, int FMT, class C, int COLL, bool SWEEP, bool BCS, class... Form>
+__global__ __launch_bounds__(256) void k_adjoint_fused(AdjParams p, Form... form) {
+  const SweepForm at = sweep_form(form...);
+  const bool pulled_in = at.pulled_in != 0, own_out = at.own_out != 0;
   constexpr LatTables T = make_tables(LAT);
   constexpr int Q = T.q;
   int x, y, z;
@@ -748,13 +784,30 @@ __global__ __launch_bounds__(256) void k_adjoint_fused(AdjParams p) {
   // the neighbour-delta flag, dL/df_out and the pulled populations.  The empty asm statement keeps
   // the compiler from sinking them below the id-dependent branches (which would cost one round
   // trip per branch); lam_in, lam_out, f_in and the delta buffers are distinct allocations.
-  const int id = p.bc_mask ? __builtin_nontemporal_load(p.bc_mask + cell) : 0;
-  const int nbf = p.nb_flag[cell];
+  int id = 0, nbf = 0;
+  if constexpr (!SWEEP) {
+    id = p.bc_mask ? __builtin_nontemporal_load(p.bc_mask + cell) : 0;
+    nbf = p.nb_flag[cell];
+  } else if constexpr (BCS) {
+    id = __builtin_nontemporal_load(p.bc_mask + cell);
+    nbf = p.nb_flag[cell];
+  }
   const C* lo = static_cast<const C*>(p.lam_out);
   C lamf[Q], fps[Q];
+  if constexpr (!SWEEP) {
 #pragma unroll
-  for (int l = 0; l < Q; ++l) lamf[l] = lo[(size_t)l * p.N + cell];
-  adj_pull<LAT, FMT, C>(p, x, y, z, fps);
+    for (int l = 0; l < Q; ++l) lamf[l] = lo[(size_t)l * p.N + cell];
+    adj_pull<LAT, FMT, C>(p, x, y, z, fps);
+  } else {
+    const int s = pulled_in ? 1 : 0;
+    const AxisShift lx(x, nx, s), ly(y, ny, s), lz(z, nz, s), fx(x, nx, -1), fy(y, ny, -1), fz(z, nz, -1);
+#pragma unroll
+    for (int l = 0; l < Q; ++l) lamf[l] = *row_at<LAT, C>(lo, (uint64_t)l * p.N, ny, nz, lx[T.c[0][l]], ly[T.c[1][l]], lz[T.c[2][l]]);
+    const typename Fmt<FMT>::raw* fin = static_cast<const typename Fmt<FMT>::raw*>(p.f_in);
+#pragma unroll
+    for (int l = 0; l < Q; ++l)
+      fps[l] = ld_pop<FMT, C>(row_at<LAT, typename Fmt<FMT>::raw>(fin, l * p.P, ny, nz, fx[T.c[0][l]], fy[T.c[1][l]], fz[T.c[2][l]]), T.w[l]);
+  }
   asm volatile("" ::: "memory");
   C* li = static_cast<C*>(p.lam_in);
   if (id == 255) {
@@ -763,7 +816,8 @@ __global__ __launch_bounds__(256) void k_adjoint_fused(AdjParams p) {
     // consistent regardless: deltas addressed to the cell are consumed like anywhere else.)
 #pragma unroll
     for (int k = 0; k < Q; ++k) {
-      const int sx = wrap1(x - T.c[0][k], nx), sy = wrap1(y - T.c[1][k], ny), sz = wrap1(z - T.c[2][k], nz);
+      int sx = wrap1(x - T.c[0][k], nx), sy = wrap1(y - T.c[1][k], ny), sz = wrap1(z - T.c[2][k], nz);
+      if (SWEEP && own_out) sx = x, sy = y, sz = z;
       li[(size_t)k * p.N + ((uint32_t)sx * ny + sy) * nz + sz] = C(0);
     }
     if (nbf) {
@@ -864,10 +918,24 @@ __global__ __launch_bounds__(256) void k_adjoint_fused(AdjParams p) {
       }
     }
   }
+  if constexpr (!SWEEP) {
 #pragma unroll
-  for (int k = 0; k < Q; ++k) {
-    const int sx = wrap1(x - T.c[0][k], nx), sy = wrap1(y - T.c[1][k], ny), sz = wrap1(z - T.c[2][k], nz);
-    li[(size_t)k * p.N + ((uint32_t)sx * ny + sy) * nz + sz] = G[k];
+    for (int k = 0; k < Q; ++k) {
+      const int sx = wrap1(x - T.c[0][k], nx), sy = wrap1(y - T.c[1][k], ny), sz = wrap1(z - T.c[2][k], nz);
+      li[(size_t)k * p.N + ((uint32_t)sx * ny + sy) * nz + sz] = G[k];
+    }
+  } else {
+    const int s = own_out ? 0 : -1;
+    const AxisShift ox(x, nx, s), oy(y, ny, s), oz(z, nz, s);
+    if (own_out && (T.d == 3 ? nz : ny) * sizeof(C) % 128 == 0) {
+#pragma unroll
+      for (int k = 0; k < Q; ++k)
+        st_stream(const_cast<C*>(row_at<LAT, C>(li, (uint64_t)k * p.N, ny, nz, ox[T.c[0][k]], oy[T.c[1][k]], oz[T.c[2][k]])), G[k]);
+    } else {
+#pragma unroll
+      for (int k = 0; k < Q; ++k)
+        *const_cast<C*>(row_at<LAT, C>(li, (uint64_t)k * p.N, ny, nz, ox[T.c[0][k]], oy[T.c[1][k]], oz[T.c[2][k]])) = G[k];
+    }
   }
   if (own_kind(kind)) {
 #pragma unroll
@@ -896,6 +964,25 @@ __global__ __launch_bounds__(256) void k_adjoint_nb_flags(AdjParams p, uint8_t* 
       const int sz = wrap(z - (T.c[2][l] + n[2]), nz);
       flag[((uint32_t)sx * ny + sy) * nz + sz] = 1;
     }
+  }
+}
+
+// Clears the carried deltas where a sweep reads them: d_own at the cells whose kind leaves deltas at
+// itself, both d_nb buffers (d_own + Q N and + 2 Q N) at flagged cells.
+template <int LAT, class C>
+__global__ __launch_bounds__(256) void k_adjoint_clear(AdjParams p, const uint8_t* flag) {
+  constexpr int Q = make_tables(LAT).q;
+  int x, y, z;
+  if (!sweep_cell(p.sw, x, y, z)) return;
+  const uint32_t cell = ((uint32_t)x * p.sw.ny + y) * p.sw.nz + z;
+  const int id = p.bc_mask[cell];
+  const bool own = id != 0 && id != 255 && own_kind(p.table[id].kind);
+  const bool nb = flag[cell] != 0;
+  C* d = static_cast<C*>(p.d_own);
+#pragma unroll
+  for (int l = 0; l < Q; ++l) {
+    if (own) d[(size_t)l * p.N + cell] = C(0);
+    if (nb) d[(size_t)(Q + l) * p.N + cell] = d[(size_t)(2 * Q + l) * p.N + cell] = C(0);
   }
 }
 
@@ -933,26 +1020,50 @@ enum AdjMode { ADJ_SPLIT = 0, ADJ_FUSED = 1, ADJ_BEGIN = 2, ADJ_FLUSH = 3 };
 template <int LAT, int FMT, class C, int COLL>
 int launch_adjoint(const AdjParams& p, hipStream_t s);
 
-// The fused path's kernels.  `ws_words` / `flag` / `lam` are used by BEGIN / FLUSH.
+// The fused path's kernels.  `flag` / `lam` are used by BEGIN / FLUSH, `pulled_in` / `own_out` by FUSED
+// (D3Q27 takes neither).
 template <int LAT, int FMT, class C, int COLL>
-int launch_adjoint_mode(const AdjParams& p, hipStream_t s, int mode, uint64_t ws_words, uint8_t* flag, void* lam) {
+int launch_adjoint_mode(const AdjParams& p, hipStream_t s, int mode, uint8_t* flag, void* lam, int pulled_in,
+                        int own_out) {
   if (mode == ADJ_SPLIT) return launch_adjoint<LAT, FMT, C, COLL>(p, s);
   if (mode == ADJ_FUSED) {
-    hipLaunchKernelGGL((k_adjoint_fused<LAT, FMT, C, COLL>), sweep_grid(p.sw), dim3(256), 0, s, p);
+    // The sweep form where it is the faster one: without a mask (FP32, us per step: 128^3 96 -> 91, 256^3
+    // 708 -> 669, 100x90x77 40 -> 33; FP64 128^3 235 -> 178) and on D2Q9 (512x256 channel 14.5 -> 11.2).
+    // The 3-D kernel with boundary paths is held to 3 waves per SIMD by its registers either way
+    // (128^3 cavity 105 plain, 110 in the sweep form), and D3Q27's spills.
+    const SweepForm form{pulled_in, own_out};
+    (void)form;
+    auto plain = [&]() {
+      hipLaunchKernelGGL((k_adjoint_fused<LAT, FMT, C, COLL, false, true>), sweep_grid(p.sw), dim3(256), 0, s, p);
+    };
+    if constexpr (LAT == XLBH_D3Q27) {
+      plain();
+    } else if (!p.bc_mask) {
+      hipLaunchKernelGGL((k_adjoint_fused<LAT, FMT, C, COLL, true, false, SweepForm>), sweep_grid(p.sw), dim3(256), 0, s, p, form);
+    } else if constexpr (LAT == XLBH_D2Q9) {
+      hipLaunchKernelGGL((k_adjoint_fused<LAT, FMT, C, COLL, true, true, SweepForm>), sweep_grid(p.sw), dim3(256), 0, s, p, form);
+    } else {
+      plain();
+    }
     XLBH_LAUNCH_CHECK();
     return 0;
   }
   if (mode == ADJ_BEGIN) {
-    const uint64_t blocks = std::min<uint64_t>((ws_words + 255) / 256, 65536);
-    hipLaunchKernelGGL(k_zero_words<0>, dim3((unsigned)blocks), dim3(256), 0, s, static_cast<uint32_t*>(p.d_own),
-                       ws_words);
+    // Without a mask nothing is carried from step to step.  (D3Q27's kernel reads the flags anyway.)
+    if (!p.bc_mask && LAT != XLBH_D3Q27) return 0;
+    const uint64_t words = ((uint64_t)p.N + 3) / 4;
+    hipLaunchKernelGGL(k_zero_words<0>, dim3((unsigned)std::min<uint64_t>((words + 255) / 256, 65536)), dim3(256), 0, s,
+                       reinterpret_cast<uint32_t*>(flag), words);
     XLBH_LAUNCH_CHECK();
     if (p.bc_mask) {
       hipLaunchKernelGGL((k_adjoint_nb_flags<LAT>), sweep_grid(p.sw), dim3(256), 0, s, p, flag);
       XLBH_LAUNCH_CHECK();
+      hipLaunchKernelGGL((k_adjoint_clear<LAT, C>), sweep_grid(p.sw), dim3(256), 0, s, p, flag);
+      XLBH_LAUNCH_CHECK();
     }
     return 0;
   }
+  if (!p.bc_mask) return 0;
   hipLaunchKernelGGL((k_adjoint_flush<LAT, C>), sweep_grid(p.sw), dim3(256), 0, s, p, static_cast<C*>(lam));
   XLBH_LAUNCH_CHECK();
   return 0;
@@ -979,25 +1090,25 @@ int launch_adjoint(const AdjParams& p, hipStream_t s) {
 // Dispatch of one lattice's reverse kernels on (store, compute, collision); each lattice is
 // instantiated in its own translation unit (adjoint_d2q9.hip, ...) so they compile in parallel.
 template <int LAT>
-int adjoint_dispatch_lat(int store, int compute, const AdjParams& p, hipStream_t s, int mode, uint64_t ws_words,
-                         uint8_t* flag, void* lam) {
+int adjoint_dispatch_lat(int store, int compute, const AdjParams& p, hipStream_t s, int mode,
+                         uint8_t* flag, void* lam, int pulled_in, int own_out) {
   // the collision is a template parameter, so each reverse kernel carries only its own collision
   auto with_coll = [&](auto K) -> int {
     constexpr int COLL = decltype(K)::value;
     if (compute == XLBH_COMPUTE_F32) {
       switch (store) {
-        case XLBH_F32: return launch_adjoint_mode<LAT, XLBH_F32, float, COLL>(p, s, mode, ws_words, flag, lam);
-        case XLBH_F16: return launch_adjoint_mode<LAT, XLBH_F16, float, COLL>(p, s, mode, ws_words, flag, lam);
-        case XLBH_BF16: return launch_adjoint_mode<LAT, XLBH_BF16, float, COLL>(p, s, mode, ws_words, flag, lam);
+        case XLBH_F32: return launch_adjoint_mode<LAT, XLBH_F32, float, COLL>(p, s, mode, flag, lam, pulled_in, own_out);
+        case XLBH_F16: return launch_adjoint_mode<LAT, XLBH_F16, float, COLL>(p, s, mode, flag, lam, pulled_in, own_out);
+        case XLBH_BF16: return launch_adjoint_mode<LAT, XLBH_BF16, float, COLL>(p, s, mode, flag, lam, pulled_in, own_out);
         case XLBH_F16_SHIFTED:
-          return launch_adjoint_mode<LAT, XLBH_F16_SHIFTED, float, COLL>(p, s, mode, ws_words, flag, lam);
+          return launch_adjoint_mode<LAT, XLBH_F16_SHIFTED, float, COLL>(p, s, mode, flag, lam, pulled_in, own_out);
         case XLBH_BF16_SHIFTED:
-          return launch_adjoint_mode<LAT, XLBH_BF16_SHIFTED, float, COLL>(p, s, mode, ws_words, flag, lam);
+          return launch_adjoint_mode<LAT, XLBH_BF16_SHIFTED, float, COLL>(p, s, mode, flag, lam, pulled_in, own_out);
       }
     } else if (compute == XLBH_COMPUTE_F64) {
       switch (store) {
-        case XLBH_F64: return launch_adjoint_mode<LAT, XLBH_F64, double, COLL>(p, s, mode, ws_words, flag, lam);
-        case XLBH_F32: return launch_adjoint_mode<LAT, XLBH_F32, double, COLL>(p, s, mode, ws_words, flag, lam);
+        case XLBH_F64: return launch_adjoint_mode<LAT, XLBH_F64, double, COLL>(p, s, mode, flag, lam, pulled_in, own_out);
+        case XLBH_F32: return launch_adjoint_mode<LAT, XLBH_F32, double, COLL>(p, s, mode, flag, lam, pulled_in, own_out);
       }
     }
     set_error("unsupported (store, compute) combination for the adjoint step");
@@ -1014,11 +1125,11 @@ int adjoint_dispatch_lat(int store, int compute, const AdjParams& p, hipStream_t
   return 1;
 }
 
-int adjoint_dispatch_d2q9(int store, int compute, const AdjParams& p, hipStream_t s, int mode, uint64_t ws_words,
-                          uint8_t* flag, void* lam);
-int adjoint_dispatch_d3q19(int store, int compute, const AdjParams& p, hipStream_t s, int mode, uint64_t ws_words,
-                           uint8_t* flag, void* lam);
-int adjoint_dispatch_d3q27(int store, int compute, const AdjParams& p, hipStream_t s, int mode, uint64_t ws_words,
-                           uint8_t* flag, void* lam);
+int adjoint_dispatch_d2q9(int store, int compute, const AdjParams& p, hipStream_t s, int mode, uint8_t* flag, void* lam,
+                          int pulled_in, int own_out);
+int adjoint_dispatch_d3q19(int store, int compute, const AdjParams& p, hipStream_t s, int mode, uint8_t* flag, void* lam,
+                          int pulled_in, int own_out);
+int adjoint_dispatch_d3q27(int store, int compute, const AdjParams& p, hipStream_t s, int mode, uint8_t* flag, void* lam,
+                          int pulled_in, int own_out);
 
 }  // namespace xlbh

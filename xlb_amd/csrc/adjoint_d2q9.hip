@@ -3,8 +3,8 @@
 #include "adjoint.hpp"
 
 namespace xlbh {
-int adjoint_dispatch_d2q9(int store, int compute, const AdjParams& p, hipStream_t s, int mode, uint64_t ws_words,
-                          uint8_t* flag, void* lam) {
-  return adjoint_dispatch_lat<XLBH_D2Q9>(store, compute, p, s, mode, ws_words, flag, lam);
+int adjoint_dispatch_d2q9(int store, int compute, const AdjParams& p, hipStream_t s, int mode, uint8_t* flag, void* lam,
+                          int pulled_in, int own_out) {
+  return adjoint_dispatch_lat<XLBH_D2Q9>(store, compute, p, s, mode, flag, lam, pulled_in, own_out);
 }
 }  // namespace xlbh
