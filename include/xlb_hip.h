@@ -207,6 +207,18 @@ int xlbh_run_known(int lattice, int collision, int store, int compute,
                    int nx, int ny, int nz, int64_t plane, double omega, double collision_param, int timestep0,
                    int n_steps, uint32_t known, void* stream);
 
+/* n_steps >= 1 steps from f_start, which is only read, through the two buffers f_a and f_b (f_b is
+ * not used by a single step); *in_b (host) tells where the newest populations are: f_a (0) or f_b
+ * (1).  The other buffer's contents are unspecified.  `known` as in xlbh_run_known.  For callers that
+ * keep f_start (a checkpoint) and would otherwise copy it before xlbh_run. */
+int xlbh_advance(int lattice, int collision, int store, int compute,
+                 const void* f_start, void* f_a, void* f_b,
+                 const uint8_t* bc_mask, const uint32_t* missing_bits,
+                 const void* aux, const xlbh_bc_desc* bc_table,
+                 int force_mode, const double* force_uniform, const void* force_field,
+                 int nx, int ny, int nz, int64_t plane, double omega, double collision_param, int timestep0,
+                 int n_steps, uint32_t known, int* in_b, void* stream);
+
 /* n_states steps from f_start, keeping every state: state j (the output of step t0 + j) is
  * written to states + j * xlbh_population_bytes(..., plane) bytes, for j = 0 .. n_states - 1.  The forward pass of a
  * checkpointed reverse sweep (xlbh_adjoint_run without XLBH_ADJ_RECOMPUTE); no counterpart in the

@@ -75,3 +75,25 @@ def test_run_and_record_equal_single_steps(shape, flow, policy, collision, force
             b0, b1 = b1, b0
             assert torch.equal(kept[t], b0), (steps, t, (kept[t] - b0).abs().max())
         assert torch.equal(a0, b0) and torch.equal(a1, b1), (steps, (a0 - b0).abs().max(), (a1 - b1).abs().max())
+
+
+@pytest.mark.parametrize("lattice,shape", [("D2Q9", (64, 50)), ("D3Q19", (64, 70, 130)), ("D3Q27", (12, 10, 14))])
+def test_advance_equals_run_and_leaves_its_start(lattice, shape):
+    import xlb_amd as xa
+
+    policy = xa.PrecisionPolicy.FP32FP32
+    vs = getattr(xa.velocity_set, lattice)(policy, xa.ComputeBackend.MI355X)
+    xa.init(velocity_set=vs, default_backend=xa.ComputeBackend.MI355X, default_precision_policy=policy)
+    grid = xa.grid.grid_factory(shape, compute_backend=xa.ComputeBackend.MI355X)
+    st = xa.operator.stepper.IncompressibleNavierStokesStepper(grid, [], collision_type="BGK")
+    f, _, bm, mm = st.prepare_fields()
+    f.mul_(1 + 0.05 * torch.rand(f.shape, generator=torch.Generator().manual_seed(1)).cuda())
+    kept = f.clone()
+    for steps in (1, 2, 3, 5, 8):
+        a, _ = st.run(f.clone(), torch.empty_like(f), bm, mm, 1.5, steps)
+        b, other = st.advance(f, torch.empty_like(f), torch.empty_like(f), bm, mm, 1.5, steps)
+        assert torch.equal(a, b) and torch.equal(f, kept) and other.data_ptr() != b.data_ptr()
+    with pytest.raises(RuntimeError):
+        st.advance(f, torch.empty_like(f), f, bm, mm, 1.5, 2)
+    with pytest.raises(RuntimeError):
+        st.advance(f, torch.empty_like(f), torch.empty_like(f), bm, mm, 1.5, 0)

@@ -55,6 +55,7 @@ _d = ctypes.c_double
 _i64 = ctypes.c_int64
 _u32 = ctypes.c_uint32
 _dp = ctypes.POINTER(ctypes.c_double)
+_ip = ctypes.POINTER(ctypes.c_int)
 _bcp = ctypes.POINTER(BcDesc)
 
 # name -> (restype, argtypes)
@@ -67,6 +68,8 @@ SIGNATURES = {
     "xlbh_run": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _dp, _vp, _i, _i, _i, _i64, _d, _d, _i, _i, _vp]),
     "xlbh_run_known": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _dp, _vp, _i, _i, _i, _i64, _d, _d, _i, _i,
                             _u32, _vp]),
+    "xlbh_advance": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _dp, _vp, _i, _i, _i, _i64, _d, _d, _i,
+                          _i, _u32, _ip, _vp]),
     "xlbh_step_slab": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _dp, _vp, _i, _i, _i, _i64, _d, _d, _i, _i,
                             _i, _vp]),
     "xlbh_stream": (_i, [_i, _i, _vp, _vp, _i, _i, _i, _i64, _vp]),

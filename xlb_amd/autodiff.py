@@ -63,7 +63,7 @@ def macroscopic_torch(f, velocity_set):
 class _Checkpoint:
     """State at a segment start.  ``mode``:
 
-    * "store": a copy in the store dtype;
+    * "store": ``f`` itself, which the caller does not write any more;
     * "bf16": the checkpoint codec of the library (xlbh_checkpoint_encode): the non-equilibrium
       part f_l - feq_l(rho, u) as bfloat16 plus rho - 1 and u as float32 ((2 Q + 4 (d + 1)) bytes per
       cell; 0.71 of an FP32 field for D3Q19);
@@ -82,7 +82,7 @@ class _Checkpoint:
         elif mode == "bf16_shifted":
             self.data = (f.float() - w).to(torch.bfloat16)
         else:
-            self.data = f.clone()
+            self.data = f
 
     def state(self, scratch, w, stepper):
         """A store-dtype tensor holding the state (``scratch`` is filled for 16-bit checkpoints)."""
@@ -112,12 +112,27 @@ class _Rollout(torch.autograd.Function):
             field = force_field.detach().to(stepper.compute_dtype, copy=True).contiguous()
             col.force_field = field
         w = torch.as_tensor(np.asarray(stepper.velocity_set.w), dtype=torch.float32, device=f0.device).reshape(-1, 1, 1, 1)
-        a = f0.detach().to(stepper.store_dtype).clone().contiguous()
-        b = torch.empty_like(a)
+        # a private copy: the first checkpoint is kept while the caller may change f0
+        a = f0.detach().to(stepper.store_dtype, copy=True, memory_format=torch.contiguous_format)
         ckpts = {}
-        for s in range(0, num_steps, every):
-            ckpts[s] = _Checkpoint(a, ckpt_mode, w, stepper)
-            a, b = stepper.run(a, b, bc_mask, missing_mask, omega, min(every, num_steps - s), timestep=s)
+        stepper._sync_state(bc_mask, missing_mask)
+        if stepper._has_solid:
+            # solid cells keep what the two buffers held: the buffers of a plain run, and copies
+            b = torch.empty_like(a)
+            for s in range(0, num_steps, every):
+                ckpts[s] = _Checkpoint(a.clone() if ckpt_mode == "store" else a, ckpt_mode, w, stepper)
+                a, b = stepper.run(a, b, bc_mask, missing_mask, omega, min(every, num_steps - s), timestep=s)
+        else:
+            # a checkpoint in the store dtype is the state itself, which the steps only read
+            free = []
+            for s in range(0, num_steps, every):
+                ckpts[s] = _Checkpoint(a, ckpt_mode, w, stepper)
+                b, c = (free.pop() if free else torch.empty_like(a) for _ in range(2))
+                new, other = stepper.advance(a, b, c, bc_mask, missing_mask, omega, min(every, num_steps - s), timestep=s)
+                free.append(other)
+                if ckpt_mode != "store":
+                    free.append(a)
+                a = new
         ctx.stepper = stepper
         ctx.masks = (bc_mask, missing_mask)
         ctx.omega = omega

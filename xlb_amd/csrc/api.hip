@@ -70,6 +70,27 @@ static int dispatch_step(int lattice, const StepCall& c) {
   return 1;
 }
 
+// The launches of a run: `per` steps each (1: k_step; 2 on D3Q19: k_step_pair; more on D2Q9:
+// k_steps_2d), as equal as they can be.
+struct Launcher {
+  int per = 1;
+  PairTiles tiles{};
+  int launches(int n) const { return (n + per - 1) / per; }
+  // steps of the next launch when `left` launches remain for `n` steps
+  int share(int n, int left) const { return (n + left - 1) / left; }
+  int operator()(int lattice, const StepCall& c, int steps, size_t state_bytes = 0) const {
+    if (steps == 1) return dispatch_step(lattice, c);
+    return lattice == XLBH_D2Q9 ? launch_steps_2d(c, steps, state_bytes) : launch_pair(lattice, c, tiles);
+  }
+};
+
+static Launcher plan_steps(int lattice, const StepCall& c, uint32_t known, int n) {
+  Launcher go;
+  if (n > 1 && steps_2d_apply(lattice, c, known)) go.per = steps_2d_best(c, n);
+  if (n > 1 && plan_pair(lattice, c, known, go.tiles)) go.per = 2;
+  return go;
+}
+
 static int validate_step(int lattice, int collision, int store, int compute, const void* f_a, const void* f_b,
                          const uint8_t* bc_mask, const uint32_t* missing_bits, const xlbh_bc_desc* bc_table,
                          int force_mode, const double* force_uniform, const void* force_field, int nx, int ny,
@@ -176,28 +197,47 @@ int xlbh_run_known(int lattice, int collision, int store, int compute, void* f_a
   // Each launch writes the buffer it does not read.  As many launches as n_steps in parity, the last
   // of them of one step, leave both buffers as n_steps one-step launches do: the newest state in
   // the buffer n_steps selects, the one before it in the other.
-  if (n_steps > 2 && steps_2d_apply(lattice, c, known)) {
-    const int per = steps_2d_best(c, n_steps - 1);
-    int launches = 1 + (n_steps - 1 + per - 1) / per;
-    launches += (launches ^ n_steps) & 1;
-    for (int k = 0, t = 0; k < launches; ++k) {
-      c.f_in = (k % 2 == 0) ? f_a : f_b;
-      c.f_out = (k % 2 == 0) ? f_b : f_a;
-      const int left = launches - 1 - k, m = left > 0 ? (n_steps - 1 - t + left - 1) / left : 1;
-      if (int e = m > 1 ? launch_steps_2d(c, m, 0) : dispatch_step(lattice, c)) return e;
-      t += m;
-    }
-    return 0;
+  const Launcher go = plan_steps(lattice, c, known, n_steps - 1);
+  int launches = n_steps > 0 ? 1 + go.launches(n_steps - 1) : 0;
+  launches += (launches ^ n_steps) & 1;
+  for (int k = 0, t = 0; k < launches; ++k) {
+    c.f_in = (k % 2 == 0) ? f_a : f_b;
+    c.f_out = (k % 2 == 0) ? f_b : f_a;
+    const int m = k < launches - 1 ? go.share(n_steps - 1 - t, launches - 1 - k) : 1;
+    if (int e = go(lattice, c, m)) return e;
+    t += m;
   }
-  PairTiles tiles;
-  int pairs = n_steps > 4 && plan_pair(lattice, c, known, tiles) ? (n_steps - 1) / 4 * 2 : 0;
-  for (int t = 0, launch = 0; t < n_steps; ++launch) {
-    c.f_in = (launch % 2 == 0) ? f_a : f_b;
-    c.f_out = (launch % 2 == 0) ? f_b : f_a;
-    const bool two = launch < pairs;
-    if (int e = two ? launch_pair(lattice, c, tiles) : dispatch_step(lattice, c)) return e;
-    t += two ? 2 : 1;
+  return 0;
+}
+
+int xlbh_advance(int lattice, int collision, int store, int compute, const void* f_start, void* f_a, void* f_b,
+                 const uint8_t* bc_mask, const uint32_t* missing_bits, const void* aux, const xlbh_bc_desc* bc_table,
+                 int force_mode, const double* force_uniform, const void* force_field, int nx, int ny, int nz,
+                 int64_t plane, double omega, double collision_param, int timestep0, int n_steps, uint32_t known,
+                 int* in_b, void* stream) {
+  (void)timestep0;
+  clear_error();
+  if (int e = validate_step(lattice, collision, store, compute, f_start, f_a, bc_mask, missing_bits, bc_table,
+                            force_mode, force_uniform, force_field, nx, ny, nz))
+    return e;
+  XLBH_REQUIRE(n_steps >= 1, "advance: n_steps must be >= 1");
+  XLBH_REQUIRE(in_b, "advance: in_b is null");
+  XLBH_REQUIRE(n_steps == 1 || (f_b && f_b != f_start && f_b != f_a),
+               "advance: more than one step needs a second buffer of its own");
+  uint64_t P;
+  if (int e = resolve_plane(lattice, store, nx, ny, nz, plane, P)) return e;
+  StepCall c{collision, store, compute, f_start, f_a, bc_mask, missing_bits, aux, bc_table,
+             force_mode, force_uniform, force_field, nx, ny, nz, P, omega, collision_param, (hipStream_t)stream};
+  const Launcher go = plan_steps(lattice, c, known, n_steps);
+  const int launches = go.launches(n_steps);
+  for (int k = 0, t = 0; k < launches; ++k) {
+    c.f_in = k == 0 ? f_start : (k % 2 == 0 ? f_b : f_a);
+    c.f_out = k % 2 == 0 ? f_a : f_b;
+    const int m = go.share(n_steps - t, launches - k);
+    if (int e = go(lattice, c, m)) return e;
+    t += m;
   }
+  *in_b = launches % 2 == 0;
   return 0;
 }
 
@@ -229,13 +269,16 @@ int xlbh_record_known(int lattice, int collision, int store, int compute, const 
   const size_t field_bytes = (size_t)xlbh_population_bytes(lattice, store, nx, ny, nz, (int64_t)P);
   StepCall c{collision, store, compute, f_start, states, bc_mask, missing_bits, aux, bc_table,
              force_mode, force_uniform, force_field, nx, ny, nz, P, omega, collision_param, (hipStream_t)stream};
-  const int per = steps_2d_apply(lattice, c, known) ? steps_2d_best(c, n_states) : 1;
-  const int launches = (n_states + per - 1) / per;
+  // (Two 3-D steps per launch that keep the first one's state too save little: 256^3 434 us per step
+  // either way, 128^3 62 against 67 us.)
+  Launcher go;
+  if (lattice == XLBH_D2Q9) go = plan_steps(lattice, c, known, n_states);
+  const int launches = go.launches(n_states);
   for (int k = 0, j = 0; k < launches; ++k) {
-    const int m = (n_states - j + launches - k - 1) / (launches - k);
+    const int m = go.share(n_states - j, launches - k);
     c.f_in = j == 0 ? f_start : static_cast<const char*>(states) + (size_t)(j - 1) * field_bytes;
     c.f_out = static_cast<char*>(states) + (size_t)j * field_bytes;
-    if (int e = m > 1 ? launch_steps_2d(c, m, field_bytes) : dispatch_step(lattice, c)) return e;
+    if (int e = go(lattice, c, m, field_bytes)) return e;
     j += m;
   }
   return 0;

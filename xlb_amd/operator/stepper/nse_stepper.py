@@ -447,3 +447,24 @@ class IncompressibleNavierStokesStepper(Stepper):
         if num_steps % 2 == 1:
             return f_1, f_0
         return f_0, f_1
+
+    def advance(self, f_start, f_a, f_b, bc_mask, missing_mask, omega, num_steps, timestep=0):
+        """``num_steps`` steps from ``f_start``, which is only read, through the buffers ``f_a`` and
+        ``f_b`` (xlbh_advance); returns (newest, other), the one of the two that holds the newest
+        populations first.  Needs no copy of a state that is kept, as ``run`` would."""
+        nx, ny, nz, plane, masks, force_mode, fu_ptr, keep, force_field = self._launch_args(f_start, f_a, bc_mask, missing_mask)
+        ext, fmt = (nx, ny, nz), self.precision_policy.store_format
+        common_plane([plane, expect_population(f_b, self.velocity_set.q, ext, "f_b", self.store_dtype, self.lattice_id, fmt)],
+                     "IncompressibleNavierStokesStepper.advance")
+        in_b = ctypes.c_int(0)
+        _lib.check(
+            _lib.lib().xlbh_advance(
+                self.lattice_id, self._collision_id(), fmt, self.compute_id,
+                _lib.ptr(f_start), _lib.ptr(f_a), _lib.ptr(f_b), *masks, force_mode, fu_ptr, _lib.ptr(force_field),
+                nx, ny, nz, plane, float(omega), self._collision_param(), int(timestep), int(num_steps), self._mask_holds,
+                ctypes.byref(in_b), _lib.stream_of(f_start),
+            ),
+            "IncompressibleNavierStokesStepper.advance",
+        )
+        _lib.mark_written(f_a, f_b)
+        return (f_b, f_a) if in_b.value else (f_a, f_b)
