@@ -227,10 +227,13 @@ __device__ __forceinline__ C ld_pop(const typename Fmt<FMT>::raw* p, double w) {
   return v;
 }
 
-template <int FMT, class C>
+template <int FMT, class C, bool NT = true>
 __device__ __forceinline__ void st_pop(typename Fmt<FMT>::raw* p, C v, double w) {
   if constexpr (Fmt<FMT>::shifted) v -= (C)w;
-  st_stream(p, to_raw<typename Fmt<FMT>::raw, C>(v));
+  if constexpr (NT)
+    st_stream(p, to_raw<typename Fmt<FMT>::raw, C>(v));
+  else
+    *p = to_raw<typename Fmt<FMT>::raw, C>(v);
 }
 
 // Macroscopic-field element types (rho, u, Pi outputs of the standalone operators).

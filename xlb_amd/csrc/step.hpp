@@ -39,6 +39,8 @@ struct StepParams {
   const int32_t* e_in;   // XLBH_I16_BLOCK: segment exponents of f_in and f_out
   int32_t* e_out;
   int x0, x1;            // the planes x0 <= x < x1 this launch updates
+  int nt;                // non-temporal stores
+  uint32_t per_xcd;      // consecutive blocks per XCD (0: blocks as the hardware deals them out)
 };
 
 // Reads of stored populations other than the pulls: the own cell's pre-stream values and the
@@ -87,15 +89,18 @@ struct PullOffsets {
   }
   // src(l) split into its wave-uniform part (the slow axes) and its per-lane part (the row axis:
   // z in 3-D, y in 2-D), for Planes::at(l, uni, lane).
-  template <int LAT>
+  // FLAT: the per-lane part is the offset in the x-plane.
+  template <int LAT, bool FLAT = false>
   __device__ __forceinline__ O uni(int l) const {
     constexpr LatTables T = make_tables(LAT);
+    if constexpr (FLAT) return xo[T.c[0][l] + 1];
     if constexpr (T.d == 3) return xo[T.c[0][l] + 1] + yo[T.c[1][l] + 1];
     return xo[T.c[0][l] + 1];
   }
-  template <int LAT>
+  template <int LAT, bool FLAT = false>
   __device__ __forceinline__ O lane(int l) const {
     constexpr LatTables T = make_tables(LAT);
+    if constexpr (FLAT) return yo[T.c[1][l] + 1] + zo[T.c[2][l] + 1];
     if constexpr (T.d == 3) return zo[T.c[2][l] + 1];
     return yo[T.c[1][l] + 1] + zo[T.c[2][l] + 1];
   }
@@ -234,10 +239,22 @@ __device__ __forceinline__ void blk_pull_exps(const StepParams& p, int xr, int y
   }
 }
 
+// The block's place in the launch grid.  The hardware deals consecutive blocks round the 8 XCDs, each
+// with an L2 of its own, so the planes a cell pulls from are mostly in another XCD's L2; regrouped,
+// each XCD takes per_xcd consecutive blocks, a slab of x-planes.  Blocks past 8 * per_xcd stay.
+__device__ __forceinline__ dim3 slab_block(uint32_t per_xcd) {
+  if (per_xcd == 0) return dim3(blockIdx.x, blockIdx.y, blockIdx.z);
+  const uint32_t lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+  const uint32_t n = lin < 8 * per_xcd ? (lin & 7) * per_xcd + (lin >> 3) : lin;
+  const uint32_t t = n / gridDim.x, z = t / gridDim.y;
+  return dim3(n - t * gridDim.x, t - z * gridDim.y, z);
+}
+
 // One thread per cell: Q pulls, the update, Q stores.  For the block format every lane of the
 // block stays to the segment reduction: lanes outside the grid read a cell of their own row and
 // write nothing, and solid cells write nothing.
-template <int LAT, int COLL, int FMT, class C, bool WIDE, bool MSEG>
+// FLAT (3-D): a block takes 256 consecutive cells of an x-plane instead of a tile of rows.
+template <int LAT, int COLL, int FMT, class C, bool WIDE, bool MSEG, bool FLAT>
 __device__ __forceinline__ void step_body(const StepParams& p) {
   constexpr LatTables T = make_tables(LAT);
   constexpr int Q = T.q;
@@ -246,8 +263,18 @@ __device__ __forceinline__ void step_body(const StepParams& p) {
   using O = typename std::conditional<WIDE, uint64_t, uint32_t>::type;
 
   int x, y, z;
-  const bool live = sweep_cell_range(p.sw, p.x0, p.x1, x, y, z);
   const int nx = p.sw.nx, ny = p.sw.ny, nz = p.sw.nz;
+  bool live;
+  if constexpr (FLAT) {
+    const dim3 b = slab_block(p.per_xcd);
+    const uint32_t i = b.x * 256u + threadIdx.x;
+    x = p.x0 + (int)b.y;
+    y = (int)(i / (uint32_t)nz);
+    z = (int)(i - (uint32_t)y * (uint32_t)nz);
+    live = y < ny;
+  } else {
+    live = sweep_cell_range(p.sw, p.x0, p.x1, x, y, z);
+  }
   if constexpr (!BLK) {
     if (!live) return;
   } else {
@@ -255,11 +282,12 @@ __device__ __forceinline__ void step_body(const StepParams& p) {
     y = min(y, ny - 1);
     z = min(z, nz - 1);
   }
-  uniform_slow_axes(T.d == 3, x, y);
+  uniform_slow_axes(T.d == 3 && !FLAT, x, y);
   const O cell = ((O)x * ny + y) * nz + z;
-  // cell = row + lane: the row's first cell (wave-uniform) and the offset along the row
-  const O row = T.d == 3 ? ((O)x * ny + y) * nz : (O)x * ny;
-  const O lane = T.d == 3 ? (O)z : (O)y;
+  // cell = row + lane: the row's first cell (wave-uniform) and the offset along the row (FLAT: the
+  // x-plane's first cell and the offset in the plane)
+  const O row = FLAT ? (O)x * ny * nz : (T.d == 3 ? ((O)x * ny + y) * nz : (O)x * ny);
+  const O lane = FLAT ? (O)y * nz + z : (T.d == 3 ? (O)z : (O)y);
   const size_t plane_bytes = (size_t)p.plane * sizeof(R);
   const Planes<R, O> fout{static_cast<const char*>(p.f_out), plane_bytes};
   PopIn<FMT, C, O> fin{{static_cast<const char*>(p.f_in), plane_bytes}, p.e_in, p.sw, 0};
@@ -293,14 +321,19 @@ __device__ __forceinline__ void step_body(const StepParams& p) {
   } else {
 #pragma unroll
     for (int l = 0; l < Q; ++l)
-      f[l] = ld_pop<FMT, C>(fin.pl.at(l, po.template uni<LAT>(l), po.template lane<LAT>(l)), T.w[l]);
+      f[l] = ld_pop<FMT, C>(fin.pl.at(l, po.template uni<LAT, FLAT>(l), po.template lane<LAT, FLAT>(l)), T.w[l]);
   }
   asm volatile("" ::: "memory");
   if constexpr (!BLK) {
     if (id == 255) return;  // solid: no update (nse_stepper.py:356-358)
     cell_update<LAT, COLL, FMT, C, O>(f, id, cell, x, y, z, p, fin);
+    if (p.nt != 0) {
 #pragma unroll
-    for (int l = 0; l < Q; ++l) st_pop<FMT, C>(fout.at_w(l, row, lane), f[l], T.w[l]);
+      for (int l = 0; l < Q; ++l) st_pop<FMT, C>(fout.at_w(l, row, lane), f[l], T.w[l]);
+    } else {
+#pragma unroll
+      for (int l = 0; l < Q; ++l) st_pop<FMT, C, false>(fout.at_w(l, row, lane), f[l], T.w[l]);
+    }
   } else {
     // Lanes that write nothing (outside the grid, or solid) run the fluid update on what they
     // pulled, unbranched, and stay out of the exponent and the stores.
@@ -340,14 +373,14 @@ constexpr unsigned kStepLdsCap = 36 * 1024;
 
 // MSEG (block format only): rows of more than one exponent segment.  Its own kernel, so each
 // form gets its own register allocation.
-template <int LAT, int COLL, int FMT, class C, bool WIDE, bool MSEG = false>
+template <int LAT, int COLL, int FMT, class C, bool WIDE, bool MSEG = false, bool FLAT = false>
 __global__ __launch_bounds__(256) void k_step(StepParams p) {
-  step_body<LAT, COLL, FMT, C, WIDE, MSEG>(p);
+  step_body<LAT, COLL, FMT, C, WIDE, MSEG, FLAT>(p);
 }
 
-template <int LAT, int COLL, int FMT, class C, bool WIDE, bool MSEG = false>
+template <int LAT, int COLL, int FMT, class C, bool WIDE, bool MSEG = false, bool FLAT = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_step_w6(StepParams p) {
-  step_body<LAT, COLL, FMT, C, WIDE, MSEG>(p);
+  step_body<LAT, COLL, FMT, C, WIDE, MSEG, FLAT>(p);
 }
 
 
@@ -392,6 +425,11 @@ StepParams step_params(const StepCall& c) {
   p.x1 = c.x1 >= 0 ? c.x1 : c.nx;
   p.N = (uint32_t)((int64_t)c.nx * c.ny * c.nz);
   p.plane = c.plane;
+  // Non-temporal stores only where rows are whole 128-byte lines: of a line shared by two rows the
+  // halves would go out one by one (D3Q19 FP32 101x83x77: 25.1 us per step, 19.9 without; 300x200x230
+  // 539 and 483; D3Q27 101x83x77 36.3 and 27.5; 256^3 the other way round, 428 and 443).
+  p.nt = (uint64_t)(c.nz > 1 ? c.nz : c.ny) * sizeof(typename Fmt<FMT>::raw) % 128 == 0;
+  p.per_xcd = 0;
   p.e_in = nullptr;
   p.e_out = nullptr;
   if constexpr (FMT == XLBH_I16_BLOCK) {
@@ -404,13 +442,37 @@ StepParams step_params(const StepCall& c) {
 
 template <int LAT, int COLL, int FMT, class C>
 int launch_step_t(const StepCall& c) {
-  const StepParams p = step_params<LAT, FMT>(c);
+  StepParams p = step_params<LAT, FMT>(c);
   // 32-bit per-lane byte offsets reach every plane of the field from its base
   const bool wide = (uint64_t)Lat<LAT>::Q * p.plane * sizeof(typename Fmt<FMT>::raw) > 0xffffffffull;
   const unsigned lds = sizeof(typename Fmt<FMT>::raw) >= 4 ? kStepLdsCap : 0u;
   constexpr bool w6 = LAT == XLBH_D3Q19 && sizeof(typename Fmt<FMT>::raw) == 2 && std::is_same<C, float>::value;
   auto launch = [&](auto mseg) {
     constexpr bool MS = decltype(mseg)::value;
+    if constexpr (Lat<LAT>::D == 3 && FMT != XLBH_I16_BLOCK) {
+      // Rows that do not fill their tiles leave lanes idle (nz = 77: 40 %, 320: 38 %) and start in the
+      // middle of cache lines; consecutive cells of the whole x-plane do not.  Grids of up to 3 M
+      // cells, whose planes the L2s and the memory-side cache still hold from the step before, go
+      // slab-wise over the XCDs.  us per step with tiles, flat, flat in slabs:
+      //   D3Q19 FP32  40x40x40 5.0 5.0 4.3, 72x32x41 5.1 6.0 4.6, 101x83x77 19.9 18.6 16.5,
+      //               100x100x320 70 67.2 68.1, 300x200x230 347 330 333, 360x360x300 1090 923 935
+      //   D3Q19 FP16  72x32x41 4.8 4.8 4.1, 101x83x77 13.7 11.8 10.6, 64x60x600 35.5 33 29.3,
+      //               200x160x200 128 91.5 98
+      //   D3Q19 FP64  72x32x41 7.9 8.5 6.4, 101x83x77 33.6 33.2 30.9
+      //   D3Q27 FP32  72x32x41 6.3 8.1 5.6, 101x83x77 27.5 25.8 22.9, 200x160x200 321 260 266
+      // Whole tiles keep the scalar row addresses (256^3 D3Q19 FP32: 428, flat 437); in slabs they gain
+      // and lose by up to a fifth (48x48x64 6.8 and 5.6, D3Q27 FP64 120x60x256 150 and 174).
+      if (!wide && (c.nz & ((1 << p.sw.lbz) - 1)) != 0) {
+        const uint32_t per_plane = (uint32_t)(((uint64_t)c.ny * c.nz + 255) / 256), planes = (uint32_t)(p.x1 - p.x0);
+        const dim3 grid(per_plane, planes);
+        if (p.N <= (3u << 20)) p.per_xcd = per_plane * planes / 8;
+        if constexpr (w6)
+          hipLaunchKernelGGL((k_step_w6<LAT, COLL, FMT, C, false, MS, true>), grid, dim3(256), lds, c.stream, p);
+        else
+          hipLaunchKernelGGL((k_step<LAT, COLL, FMT, C, false, MS, true>), grid, dim3(256), lds, c.stream, p);
+        return;
+      }
+    }
     if (wide)
       hipLaunchKernelGGL((k_step<LAT, COLL, FMT, C, true, MS>), sweep_grid_range(p.sw, p.x0, p.x1), dim3(256), lds, c.stream, p);
     else if constexpr (w6)
