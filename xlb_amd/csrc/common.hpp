@@ -220,9 +220,9 @@ __device__ __forceinline__ void st_stream(R* p, R v) {
 }
 
 // Load population l (weight w) of format FMT as compute type C.
-template <int FMT, class C>
+template <int FMT, class C, bool NT = false>
 __device__ __forceinline__ C ld_pop(const typename Fmt<FMT>::raw* p, double w) {
-  C v = raw_to<typename Fmt<FMT>::raw, C>(ld_stream(p));
+  C v = raw_to<typename Fmt<FMT>::raw, C>(NT ? __builtin_nontemporal_load(p) : ld_stream(p));
   if constexpr (Fmt<FMT>::shifted) v += (C)w;
   return v;
 }
@@ -308,6 +308,17 @@ __device__ __forceinline__ bool sweep_cell_range(const Sweep& s, int x0, int x1,
   const bool in = sweep_cell_of(s, blockIdx.x, blockIdx.y, blockIdx.z, x, y, z);
   x += x0;
   return in && x < x1;
+}
+
+// The block's place in the launch grid.  The hardware deals consecutive blocks round the 8 XCDs, each
+// with an L2 of its own, so the planes a cell pulls from are mostly in another XCD's L2; regrouped,
+// each XCD takes per_xcd consecutive blocks, a slab of x-planes.  Blocks past 8 * per_xcd stay.
+__device__ __forceinline__ dim3 slab_block(uint32_t per_xcd) {
+  if (per_xcd == 0) return dim3(blockIdx.x, blockIdx.y, blockIdx.z);
+  const uint32_t lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+  const uint32_t n = lin < 8 * per_xcd ? (lin & 7) * per_xcd + (lin >> 3) : lin;
+  const uint32_t t = n / gridDim.x, z = t / gridDim.y;
+  return dim3(n - t * gridDim.x, t - z * gridDim.y, z);
 }
 
 __device__ __forceinline__ int wrap(int v, int n) {

@@ -9,11 +9,31 @@
 #include "common.hpp"
 
 namespace xlbh {
-
 template <class T>
 struct Grad {
   T xx, xy, xz, yx, yy, yz, zx, zy, zz;  // d u_a / d b as u_a_db
 };
+
+// How the stencils run on a velocity of `bytes`.
+// nt, from 16 MB on: the outputs go out past the caches and leave them to the velocity, which the
+// moments kernel has just written (moments, vorticity and Q-criterion together, FP32 256^3: 505 and
+// 480 us, 300x200x230 495 and 458; below, the outputs fit too, 250x131x40 45.4 and 46.2).
+// slabs, from 16 to 256 MB: every velocity row is read by five rows' blocks, which then share an L2;
+// it pays while the memory-side cache (256 MB) holds the velocity (us without and with: FP32 256^3 480
+// and 471, 128^3 62 and 57, 300x200x230 457 and 442; FP64 300x200x230, 331 MB, 917 and 934;
+// Q-criterion alone, FP32 101x83x77, 8 MB, 7.0 and 7.4).
+struct StencilForm {
+  bool nt, slabs;
+};
+inline StencilForm stencil_form(uint64_t bytes) {
+  return StencilForm{bytes >= (16ull << 20), bytes >= (16ull << 20) && bytes <= (256ull << 20)};
+}
+
+// sweep_cell for blocks regrouped by slab_block
+__device__ __forceinline__ bool stencil_cell(const Sweep& sw, uint32_t per_xcd, int& x, int& y, int& z) {
+  const dim3 b = slab_block(per_xcd);
+  return sweep_cell_of(sw, b.x, b.y, b.z, x, y, z);
+}
 
 // Returns false when the cell is on the domain edge or, with MASK, next to a boundary cell.  x and
 // y are wave-uniform (uniform_slow_axes), so every neighbour's address is a scalar row base plus
@@ -58,11 +78,21 @@ __device__ __forceinline__ bool central_gradient(const T* u, const uint8_t* bc_m
   return true;
 }
 
-template <class T, class O, bool MASK>
+template <bool NT, class T>
+__device__ __forceinline__ void st_out(T* p, T v) {
+  if constexpr (NT)
+    st_stream(p, v);
+  else
+    *p = v;
+}
+
+// Bound by the velocity's reads (with the moments before them, FP32 256^3 cavity: 512 -> 454 us).
+template <class T, class O, bool MASK, bool NT>
 __global__ __launch_bounds__(256) void k_vorticity(const T* __restrict__ u, const uint8_t* __restrict__ bc_mask,
-                                                   T* __restrict__ vort, T* __restrict__ mag, Sweep sw) {
+                                                   T* __restrict__ vort, T* __restrict__ mag, Sweep sw,
+                                                   uint32_t per_xcd) {
   int x, y, z;
-  if (!sweep_cell(sw, x, y, z)) return;
+  if (!stencil_cell(sw, per_xcd, x, y, z)) return;
   uniform_slow_axes(true, x, y);
   const uint64_t N = (uint64_t)sw.nx * sw.ny * sw.nz;
   Grad<T> g;
@@ -73,17 +103,18 @@ __global__ __launch_bounds__(256) void k_vorticity(const T* __restrict__ u, cons
   const T vz = g.yx - g.xy;
   const Planes<T, O> vo{reinterpret_cast<const char*>(vort), (size_t)N * sizeof(T)};
   const Planes<T, O> mo{reinterpret_cast<const char*>(mag), 0};
-  *vo.at_w(0, row, (O)z) = vx;
-  *vo.at_w(1, row, (O)z) = vy;
-  *vo.at_w(2, row, (O)z) = vz;
-  *mo.at_w(0, row, (O)z) = sqrt(vx * vx + vy * vy + vz * vz);
+  st_out<NT>(vo.at_w(0, row, (O)z), vx);
+  st_out<NT>(vo.at_w(1, row, (O)z), vy);
+  st_out<NT>(vo.at_w(2, row, (O)z), vz);
+  st_out<NT>(mo.at_w(0, row, (O)z), sqrt(vx * vx + vy * vy + vz * vz));
 }
 
-template <class T, class O, bool MASK>
+template <class T, class O, bool MASK, bool NT>
 __global__ __launch_bounds__(256) void k_q_criterion(const T* __restrict__ u, const uint8_t* __restrict__ bc_mask,
-                                                     T* __restrict__ norm_mu, T* __restrict__ q, Sweep sw) {
+                                                     T* __restrict__ norm_mu, T* __restrict__ q, Sweep sw,
+                                                     uint32_t per_xcd) {
   int x, y, z;
-  if (!sweep_cell(sw, x, y, z)) return;
+  if (!stencil_cell(sw, per_xcd, x, y, z)) return;
   uniform_slow_axes(true, x, y);
   const uint64_t N = (uint64_t)sw.nx * sw.ny * sw.nz;
   Grad<T> g;
@@ -100,22 +131,30 @@ __global__ __launch_bounds__(256) void k_q_criterion(const T* __restrict__ u, co
   const T oo = zero * zero + o01 * o01 + o02 * o02 + (-o01) * (-o01) + zero * zero + o12 * o12 + (-o02) * (-o02) +
                (-o12) * (-o12) + zero * zero;
   const Planes<T, O> no{reinterpret_cast<const char*>(norm_mu), 0}, qo{reinterpret_cast<const char*>(q), 0};
-  *no.at_w(0, row, (O)z) = mu;
-  *qo.at_w(0, row, (O)z) = half * (oo - ss);
+  st_out<NT>(no.at_w(0, row, (O)z), mu);
+  st_out<NT>(qo.at_w(0, row, (O)z), half * (oo - ss));
 }
 
-// Calls fn(T{}, O{}, integral_constant<bool, MASK>{}) for the field's element type, the offset
+// Calls fn(T{}, O{}, integral_constant<bool, MASK>{}, integral_constant<bool, NT>{}, per_xcd) for the field's element type, the offset
 // type its three velocity planes need and whether a boundary mask is given; false for an unknown
 // field type.
 template <class Fn>
-bool with_stencil_types(int field, uint64_t N, bool mask, Fn&& fn) {
+bool with_stencil_types(int field, const Sweep& sw, bool mask, Fn&& fn) {
   auto pick = [&](auto t) {
     using T = decltype(t);
-    const bool narrow = 3 * N * sizeof(T) <= 0xffffffffull;
-    if (narrow && mask) fn(t, uint32_t{}, std::true_type{});
-    else if (narrow) fn(t, uint32_t{}, std::false_type{});
-    else if (mask) fn(t, uint64_t{}, std::true_type{});
-    else fn(t, uint64_t{}, std::false_type{});
+    const uint64_t bytes = 3 * (uint64_t)sw.nx * sw.ny * sw.nz * sizeof(T);
+    const StencilForm form = stencil_form(bytes);
+    const dim3 g = sweep_grid(sw);
+    const uint32_t per_xcd = form.slabs ? g.x * g.y * g.z / 8 : 0;
+    const bool narrow = bytes <= 0xffffffffull;
+    auto go = [&](auto o, auto m) {
+      if (form.nt) fn(t, o, m, std::true_type{}, per_xcd);
+      else fn(t, o, m, std::false_type{}, per_xcd);
+    };
+    if (narrow && mask) go(uint32_t{}, std::true_type{});
+    else if (narrow) go(uint32_t{}, std::false_type{});
+    else if (mask) go(uint64_t{}, std::true_type{});
+    else go(uint64_t{}, std::false_type{});
     return true;
   };
   if (field == XLBH_FIELD_F32) return pick(float{});
@@ -138,11 +177,10 @@ int xlbh_vorticity(int field, const void* u, const uint8_t* bc_mask, void* vorti
   XLBH_REQUIRE(u && vorticity && magnitude, "vorticity needs u, vorticity and magnitude");
   const Sweep sw = make_sweep(nx, ny, nz);
   hipStream_t s = (hipStream_t)stream;
-  const uint64_t N = (uint64_t)nx * ny * nz;
-  const bool launched = with_stencil_types(field, N, bc_mask != nullptr, [&](auto t, auto o, auto m) {
+  const bool launched = with_stencil_types(field, sw, bc_mask != nullptr, [&](auto t, auto o, auto m, auto nt, uint32_t per_xcd) {
     using T = decltype(t);
-    hipLaunchKernelGGL((k_vorticity<T, decltype(o), decltype(m)::value>), sweep_grid(sw), dim3(256), 0, s,
-                       (const T*)u, bc_mask, (T*)vorticity, (T*)magnitude, sw);
+    hipLaunchKernelGGL((k_vorticity<T, decltype(o), decltype(m)::value, decltype(nt)::value>), sweep_grid(sw), dim3(256), 0, s,
+                       (const T*)u, bc_mask, (T*)vorticity, (T*)magnitude, sw, per_xcd);
   });
   if (!launched) {
     set_error("vorticity supports float32 and float64 fields");
@@ -161,11 +199,10 @@ int xlbh_q_criterion(int field, const void* u, const uint8_t* bc_mask, void* nor
   XLBH_REQUIRE(u && norm_mu && q, "q_criterion needs u, norm_mu and q");
   const Sweep sw = make_sweep(nx, ny, nz);
   hipStream_t s = (hipStream_t)stream;
-  const uint64_t N = (uint64_t)nx * ny * nz;
-  const bool launched = with_stencil_types(field, N, bc_mask != nullptr, [&](auto t, auto o, auto m) {
+  const bool launched = with_stencil_types(field, sw, bc_mask != nullptr, [&](auto t, auto o, auto m, auto nt, uint32_t per_xcd) {
     using T = decltype(t);
-    hipLaunchKernelGGL((k_q_criterion<T, decltype(o), decltype(m)::value>), sweep_grid(sw), dim3(256), 0, s,
-                       (const T*)u, bc_mask, (T*)norm_mu, (T*)q, sw);
+    hipLaunchKernelGGL((k_q_criterion<T, decltype(o), decltype(m)::value, decltype(nt)::value>), sweep_grid(sw), dim3(256), 0, s,
+                       (const T*)u, bc_mask, (T*)norm_mu, (T*)q, sw, per_xcd);
   });
   if (!launched) {
     set_error("q_criterion supports float32 and float64 fields");

@@ -239,17 +239,6 @@ __device__ __forceinline__ void blk_pull_exps(const StepParams& p, int xr, int y
   }
 }
 
-// The block's place in the launch grid.  The hardware deals consecutive blocks round the 8 XCDs, each
-// with an L2 of its own, so the planes a cell pulls from are mostly in another XCD's L2; regrouped,
-// each XCD takes per_xcd consecutive blocks, a slab of x-planes.  Blocks past 8 * per_xcd stay.
-__device__ __forceinline__ dim3 slab_block(uint32_t per_xcd) {
-  if (per_xcd == 0) return dim3(blockIdx.x, blockIdx.y, blockIdx.z);
-  const uint32_t lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-  const uint32_t n = lin < 8 * per_xcd ? (lin & 7) * per_xcd + (lin >> 3) : lin;
-  const uint32_t t = n / gridDim.x, z = t / gridDim.y;
-  return dim3(n - t * gridDim.x, t - z * gridDim.y, z);
-}
-
 // One thread per cell: Q pulls, the update, Q stores.  For the block format every lane of the
 // block stays to the segment reduction: lanes outside the grid read a cell of their own row and
 // write nothing, and solid cells write nothing.
