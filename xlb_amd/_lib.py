@@ -148,9 +148,12 @@ def require_cuda(*tensors):
 
 
 def stream_of(t=None):
-    """hipStream_t (as void*) of torch's current stream on the tensor's device."""
-    index = t.device.index if t is not None else None
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    """hipStream_t (as void*) of torch's current stream on the tensor's device; a tensor that is not
+    on a GPU has none (its pointer must not reach a kernel)."""
+    if t is None:
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    require_cuda(t)
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def doubles(values):

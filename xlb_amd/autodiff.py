@@ -115,7 +115,8 @@ class _Rollout(torch.autograd.Function):
         # a private copy: the first checkpoint is kept while the caller may change f0
         a = f0.detach().to(stepper.store_dtype, copy=True, memory_format=torch.contiguous_format)
         ckpts = {}
-        stepper._sync_state(bc_mask, missing_mask)
+        # the state of the masks, and the checks of a step: the first checkpoint is encoded before one
+        stepper._launch_args(a, None, bc_mask, missing_mask)
         if stepper._has_solid:
             # solid cells keep what the two buffers held: the buffers of a plain run, and copies
             b = torch.empty_like(a)
