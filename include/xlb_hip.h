@@ -220,7 +220,9 @@ int xlbh_advance(int lattice, int collision, int store, int compute,
                  int n_steps, uint32_t known, int* in_b, void* stream);
 
 /* n_states steps from f_start, keeping every state: state j (the output of step t0 + j) is
- * written to states + j * xlbh_population_bytes(..., plane) bytes, for j = 0 .. n_states - 1.  The forward pass of a
+ * written to states + j * xlbh_population_bytes(..., plane) bytes, for j = 0 .. n_states - 1.
+ * f_start may be one of the states but the first (a buffer that is recorded into again and again
+ * starts from its last).  The forward pass of a
  * checkpointed reverse sweep (xlbh_adjoint_run without XLBH_ADJ_RECOMPUTE); no counterpart in the
  * reference, whose tape keeps the segment's states itself. */
 int xlbh_record(int lattice, int collision, int store, int compute, const void* f_start, void* states,

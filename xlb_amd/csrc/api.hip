@@ -254,7 +254,7 @@ int xlbh_record_known(int lattice, int collision, int store, int compute, const 
                 const uint8_t* bc_mask, const uint32_t* missing_bits, const void* aux, const xlbh_bc_desc* bc_table,
                 int force_mode, const double* force_uniform, const void* force_field, int nx, int ny, int nz,
                 int64_t plane, double omega, double collision_param, int timestep0, int n_states,
-                      uint32_t known, void* stream) {
+                uint32_t known, void* stream) {
   (void)timestep0;
   clear_error();
   XLBH_REQUIRE(n_states >= 0, "n_states must be >= 0");
@@ -273,9 +273,13 @@ int xlbh_record_known(int lattice, int collision, int store, int compute, const 
   // either way, 128^3 62 against 67 us.)
   Launcher go;
   if (lattice == XLBH_D2Q9) go = plan_steps(lattice, c, known, n_states);
-  const int launches = go.launches(n_states);
+  // A recording may start from one of the states it overwrites, which its first step reads: a launch
+  // of several steps would write that state while other blocks still read it.
+  const uintptr_t at = (uintptr_t)f_start, kept = (uintptr_t)states;
+  const int first = at < kept + n_states * field_bytes && kept < at + field_bytes ? 1 : 0;
+  const int launches = first + go.launches(n_states - first);
   for (int k = 0, j = 0; k < launches; ++k) {
-    const int m = go.share(n_states - j, launches - k);
+    const int m = k < first ? 1 : go.share(n_states - j, launches - k);
     c.f_in = j == 0 ? f_start : static_cast<const char*>(states) + (size_t)(j - 1) * field_bytes;
     c.f_out = static_cast<char*>(states) + (size_t)j * field_bytes;
     if (int e = go(lattice, c, m, field_bytes)) return e;
