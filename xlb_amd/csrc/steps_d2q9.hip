@@ -9,12 +9,16 @@ static int64_t steps_2d_blocks(const StepCall& c, int steps) {
 }
 
 bool steps_2d_apply(int lattice, const StepCall& c, uint32_t known) {
-  // Solid cells keep what the output buffer held, and an outflow source two cells away may lie
-  // outside the block.
-  if (lattice != XLBH_D2Q9 || (c.bc_mask && (known & (XLBH_MASK_SOLID | XLBH_MASK_FAR_OUTFLOW)) != 0)) return false;
+  // What k_steps_2d implements.  Solid cells are not among them (they keep what the output buffer
+  // held), nor outflow sources two cells away (they may lie outside the block).
+  constexpr uint32_t kinds = 1u << XLBH_BC_NONE | 1u << XLBH_BC_EQUILIBRIUM | 1u << XLBH_BC_HALFWAY_BB |
+                             1u << XLBH_BC_FULLWAY_BB | 1u << XLBH_BC_DO_NOTHING | 1u << XLBH_BC_ZOUHE_VELOCITY |
+                             1u << XLBH_BC_ZOUHE_PRESSURE | 1u << XLBH_BC_REGULARIZED_VELOCITY |
+                             1u << XLBH_BC_REGULARIZED_PRESSURE | 1u << XLBH_BC_EXTRAPOLATION_OUTFLOW;
+  if (lattice != XLBH_D2Q9 || (c.bc_mask && (known & ~kinds) != 0)) return false;
   const bool f32 = c.store == XLBH_F32 && c.compute == XLBH_COMPUTE_F32;
   const bool f64 = c.store == XLBH_F64 && c.compute == XLBH_COMPUTE_F64;
-  return (f32 || f64) && true && steps_2d_blocks(c, kMaxSteps2d) < (int64_t)1 << 31;
+  return (f32 || f64) && steps_2d_blocks(c, kMaxSteps2d) < (int64_t)1 << 31;
 }
 
 // A launch takes about 6 us and 1.5 us per step (the channel's; a periodic box less of both) for
