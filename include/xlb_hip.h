@@ -419,8 +419,13 @@ int xlbh_adjoint_step(int lattice, int collision, int store, int compute,
  *   (one kernel per step; boundary contributions are carried to the next reverse step in the
  *   workspace instead of being added by a second kernel).  A sweep over several segments passes
  *   the same workspace to every call, with XLBH_ADJ_BEGIN on its first call (clears it) and
- *   XLBH_ADJ_END on its last (adds the carried contributions into the result).  Calls that share
- *   one workspace must not run concurrently. */
+ *   XLBH_ADJ_END on its last (adds the carried contributions into the result).  XLBH_ADJ_ONE_MASK on
+ *   every call says that they all have the same mask, missing bits and table, which saves most of the
+ *   clearing and the search for carried contributions where there is no mask (a single call with both
+ *   BEGIN and END says so by itself).  Without it the mask of an earlier segment may hold boundary
+ *   cells (not outflows) that a later one's does not; the other way round, and for outflows, the
+ *   contributions carried across would be lost.  Calls that share one workspace must not run
+ *   concurrently. */
 int xlbh_adjoint_run(int lattice, int collision, int store, int compute,
                      const void* f_ckpt, void* states, void* lam_a, void* lam_b,
                      const uint8_t* bc_mask, const uint32_t* missing_bits,
@@ -433,6 +438,7 @@ int xlbh_adjoint_run(int lattice, int collision, int store, int compute,
 #define XLBH_ADJ_RECOMPUTE 1
 #define XLBH_ADJ_BEGIN 2
 #define XLBH_ADJ_END 4
+#define XLBH_ADJ_ONE_MASK 8
 
 /* xlbh_adjoint_run for a caller that knows what its boundary mask holds (`known` as in
  * xlbh_run_known).  XLBH_MASK_SOLID set makes it check the mask as xlbh_adjoint_run does; without it

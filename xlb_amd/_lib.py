@@ -32,7 +32,7 @@ BC_REGULARIZED_PRESSURE = 8
 BC_EXTRAPOLATION_OUTFLOW = 9
 BC_GRADS_APPROXIMATION = 10
 FORCE_NONE, FORCE_UNIFORM, FORCE_FIELD = 0, 1, 2
-ADJ_RECOMPUTE, ADJ_BEGIN, ADJ_END = 1, 2, 4
+ADJ_RECOMPUTE, ADJ_BEGIN, ADJ_END, ADJ_ONE_MASK = 1, 2, 4, 8
 MASK_SOLID, MASK_FAR_OUTFLOW = 1 << 30, 1 << 29
 
 ABI_VERSION = 4

@@ -195,7 +195,7 @@ class _Rollout(torch.autograd.Function):
                         f_next = record(idx + 1)
                 out = st.adjoint_run(f_cur, states[idx % nbuf], lam_a, lam_b, bc_mask, missing_mask, ctx.omega,
                                      length, timestep=s, grad_force=grad_force, recompute=False, workspace=workspace,
-                                     begin=(idx == 0), end=(idx == len(starts) - 1))
+                                     begin=(idx == 0), end=(idx == len(starts) - 1), one_mask=True)
                 if out is lam_b:
                     lam_a, lam_b = lam_b, lam_a
                 if idx + 1 < len(starts):

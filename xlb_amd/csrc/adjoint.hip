@@ -8,13 +8,12 @@
 using namespace xlbh;
 
 static int adjoint_dispatch(int lattice, int store, int compute, const AdjParams& p, hipStream_t s,
-                            int mode = ADJ_SPLIT, uint8_t* flag = nullptr, void* lam = nullptr, int pulled_in = 0,
-                            int own_out = 0) {
+                            const AdjCall& call = AdjCall()) {
   compute = arith_compute(compute);  // the reverse kernels of the deviation form are the FP32 ones
   switch (lattice) {
-    case XLBH_D2Q9: return adjoint_dispatch_d2q9(store, compute, p, s, mode, flag, lam, pulled_in, own_out);
-    case XLBH_D3Q19: return adjoint_dispatch_d3q19(store, compute, p, s, mode, flag, lam, pulled_in, own_out);
-    case XLBH_D3Q27: return adjoint_dispatch_d3q27(store, compute, p, s, mode, flag, lam, pulled_in, own_out);
+    case XLBH_D2Q9: return adjoint_dispatch_d2q9(store, compute, p, s, call);
+    case XLBH_D3Q19: return adjoint_dispatch_d3q19(store, compute, p, s, call);
+    case XLBH_D3Q27: return adjoint_dispatch_d3q27(store, compute, p, s, call);
   }
   set_error("unknown lattice id");
   return 1;
@@ -173,16 +172,23 @@ extern "C" int xlbh_adjoint_run_known(int lattice, int collision, int store, int
     p.nb_flag = flag;
     return p;
   };
+  AdjCall call;
+  constexpr int whole = XLBH_ADJ_BEGIN | XLBH_ADJ_END;
+  call.one_mask = (flags & XLBH_ADJ_ONE_MASK) != 0 || (flags & whole) == whole;
+  call.flag = flag;
   if (ws && (flags & XLBH_ADJ_BEGIN)) {
     const AdjParams p = fused_params(f_ckpt, lam_a, lam_b, timestep0);
-    if (int e = adjoint_dispatch(lattice, store, compute, p, s, ADJ_BEGIN, flag)) return e;
+    call.mode = ADJ_BEGIN;
+    if (int e = adjoint_dispatch(lattice, store, compute, p, s, call)) return e;
   }
   for (int j = n_steps - 1; j >= 0; --j) {
     if (ws) {
       const AdjParams p = fused_params(state(j), cur, nxt, timestep0 + j);
       // the first step reads and the last one writes plain dL/df; in between it stays where it was made
-      if (int e = adjoint_dispatch(lattice, store, compute, p, s, ADJ_FUSED, nullptr, nullptr, j != n_steps - 1, j != 0))
-        return e;
+      call.mode = ADJ_FUSED;
+      call.pulled_in = j != n_steps - 1;
+      call.own_out = j != 0;
+      if (int e = adjoint_dispatch(lattice, store, compute, p, s, call)) return e;
     } else {
       const AdjParams p = adjoint_params(collision, collision_param, state(j), cur, nxt, bc_mask, missing_bits, aux,
                                          bc_table, bc_cells, n_bc_cells, force_mode, force_uniform, force_field,
@@ -195,7 +201,9 @@ extern "C" int xlbh_adjoint_run_known(int lattice, int collision, int store, int
   }
   if (ws && (flags & XLBH_ADJ_END)) {
     const AdjParams p = fused_params(f_ckpt, nullptr, nullptr, timestep0);
-    if (int e = adjoint_dispatch(lattice, store, compute, p, s, ADJ_FLUSH, nullptr, cur)) return e;
+    call.mode = ADJ_FLUSH;
+    call.lam = cur;
+    if (int e = adjoint_dispatch(lattice, store, compute, p, s, call)) return e;
   }
   return 0;
 }

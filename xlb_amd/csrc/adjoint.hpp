@@ -1017,54 +1017,69 @@ __global__ __launch_bounds__(256) void k_zero_words(uint32_t* p, uint64_t n) {
 
 enum AdjMode { ADJ_SPLIT = 0, ADJ_FUSED = 1, ADJ_BEGIN = 2, ADJ_FLUSH = 3 };
 
+// What a launch of the reverse sweep is to do.
+struct AdjCall {
+  AdjMode mode = ADJ_SPLIT;
+  bool one_mask = false;               // every call of the sweep has the same masks (fused path)
+  uint8_t* flag = nullptr;             // ADJ_BEGIN: the flag bytes of the workspace
+  void* lam = nullptr;                 // ADJ_FLUSH: dL/df
+  int pulled_in = 0, own_out = 0;      // ADJ_FUSED: the form of dL/df read and written (D3Q27 takes neither)
+};
+
 template <int LAT, int FMT, class C, int COLL>
 int launch_adjoint(const AdjParams& p, hipStream_t s);
 
-// The fused path's kernels.  `flag` / `lam` are used by BEGIN / FLUSH, `pulled_in` / `own_out` by FUSED
-// (D3Q27 takes neither).
+// The fused path's kernels.  Where the calls of a sweep may have different masks (a wall that is there
+// in some segments only), a step may read deltas that an earlier call's mask gives no reason for: the
+// whole workspace is cleared, and steps without a mask look for carried deltas all the same.
 template <int LAT, int FMT, class C, int COLL>
-int launch_adjoint_mode(const AdjParams& p, hipStream_t s, int mode, uint8_t* flag, void* lam, int pulled_in,
-                        int own_out) {
-  if (mode == ADJ_SPLIT) return launch_adjoint<LAT, FMT, C, COLL>(p, s);
-  if (mode == ADJ_FUSED) {
+int launch_adjoint_mode(const AdjParams& p, hipStream_t s, const AdjCall& call) {
+  if (call.mode == ADJ_SPLIT) return launch_adjoint<LAT, FMT, C, COLL>(p, s);
+  if (call.mode == ADJ_FUSED) {
     // The sweep form where it is the faster one: without a mask (FP32, us per step: 128^3 96 -> 91, 256^3
     // 708 -> 669, 100x90x77 40 -> 33; FP64 128^3 235 -> 178) and on D2Q9 (512x256 channel 14.5 -> 11.2).
     // The 3-D kernel with boundary paths is held to 3 waves per SIMD by its registers either way
     // (128^3 cavity 105 plain, 110 in the sweep form), and D3Q27's spills.
-    const SweepForm form{pulled_in, own_out};
+    const SweepForm form{call.pulled_in, call.own_out};
     (void)form;
     auto plain = [&]() {
       hipLaunchKernelGGL((k_adjoint_fused<LAT, FMT, C, COLL, false, true>), sweep_grid(p.sw), dim3(256), 0, s, p);
     };
     if constexpr (LAT == XLBH_D3Q27) {
       plain();
-    } else if (!p.bc_mask) {
+    } else if (!p.bc_mask && call.one_mask) {
       hipLaunchKernelGGL((k_adjoint_fused<LAT, FMT, C, COLL, true, false, SweepForm>), sweep_grid(p.sw), dim3(256), 0, s, p, form);
-    } else if constexpr (LAT == XLBH_D2Q9) {
-      hipLaunchKernelGGL((k_adjoint_fused<LAT, FMT, C, COLL, true, true, SweepForm>), sweep_grid(p.sw), dim3(256), 0, s, p, form);
+    } else if (LAT == XLBH_D2Q9 && p.bc_mask) {
+      if constexpr (LAT == XLBH_D2Q9)
+        hipLaunchKernelGGL((k_adjoint_fused<LAT, FMT, C, COLL, true, true, SweepForm>), sweep_grid(p.sw), dim3(256), 0, s, p, form);
     } else {
       plain();
     }
     XLBH_LAUNCH_CHECK();
     return 0;
   }
-  if (mode == ADJ_BEGIN) {
-    // Without a mask nothing is carried from step to step.  (D3Q27's kernel reads the flags anyway.)
-    if (!p.bc_mask && LAT != XLBH_D3Q27) return 0;
-    const uint64_t words = ((uint64_t)p.N + 3) / 4;
+  if (call.mode == ADJ_BEGIN) {
+    // With one mask, and none at that, nothing is carried from step to step.  (D3Q27's kernel reads the
+    // flags anyway.)
+    if (call.one_mask && !p.bc_mask && LAT != XLBH_D3Q27) return 0;
+    uint32_t* from = call.one_mask ? reinterpret_cast<uint32_t*>(call.flag) : static_cast<uint32_t*>(p.d_own);
+    const uint64_t bytes = (uint64_t)p.N + (call.one_mask ? 0 : 3ull * Lat<LAT>::Q * p.N * sizeof(C));
+    const uint64_t words = (bytes + 3) / 4;
     hipLaunchKernelGGL(k_zero_words<0>, dim3((unsigned)std::min<uint64_t>((words + 255) / 256, 65536)), dim3(256), 0, s,
-                       reinterpret_cast<uint32_t*>(flag), words);
+                       from, words);
     XLBH_LAUNCH_CHECK();
     if (p.bc_mask) {
-      hipLaunchKernelGGL((k_adjoint_nb_flags<LAT>), sweep_grid(p.sw), dim3(256), 0, s, p, flag);
+      hipLaunchKernelGGL((k_adjoint_nb_flags<LAT>), sweep_grid(p.sw), dim3(256), 0, s, p, call.flag);
       XLBH_LAUNCH_CHECK();
-      hipLaunchKernelGGL((k_adjoint_clear<LAT, C>), sweep_grid(p.sw), dim3(256), 0, s, p, flag);
+    }
+    if (p.bc_mask && call.one_mask) {
+      hipLaunchKernelGGL((k_adjoint_clear<LAT, C>), sweep_grid(p.sw), dim3(256), 0, s, p, call.flag);
       XLBH_LAUNCH_CHECK();
     }
     return 0;
   }
-  if (!p.bc_mask) return 0;
-  hipLaunchKernelGGL((k_adjoint_flush<LAT, C>), sweep_grid(p.sw), dim3(256), 0, s, p, static_cast<C*>(lam));
+  if (!p.bc_mask && call.one_mask) return 0;
+  hipLaunchKernelGGL((k_adjoint_flush<LAT, C>), sweep_grid(p.sw), dim3(256), 0, s, p, static_cast<C*>(call.lam));
   XLBH_LAUNCH_CHECK();
   return 0;
 }
@@ -1090,32 +1105,31 @@ int launch_adjoint(const AdjParams& p, hipStream_t s) {
 // Dispatch of one lattice's reverse kernels on (store, compute, collision); each lattice is
 // instantiated in its own translation unit (adjoint_d2q9.hip, ...) so they compile in parallel.
 template <int LAT>
-int adjoint_dispatch_lat(int store, int compute, const AdjParams& p, hipStream_t s, int mode,
-                         uint8_t* flag, void* lam, int pulled_in, int own_out) {
+int adjoint_dispatch_lat(int store, int compute, const AdjParams& p, hipStream_t s, const AdjCall& call) {
   // the collision is a template parameter, so each reverse kernel carries only its own collision
   auto with_coll = [&](auto K) -> int {
     constexpr int COLL = decltype(K)::value;
     if (compute == XLBH_COMPUTE_F32) {
       switch (store) {
-        case XLBH_F32: return launch_adjoint_mode<LAT, XLBH_F32, float, COLL>(p, s, mode, flag, lam, pulled_in, own_out);
-        case XLBH_F16: return launch_adjoint_mode<LAT, XLBH_F16, float, COLL>(p, s, mode, flag, lam, pulled_in, own_out);
-        case XLBH_BF16: return launch_adjoint_mode<LAT, XLBH_BF16, float, COLL>(p, s, mode, flag, lam, pulled_in, own_out);
+        case XLBH_F32: return launch_adjoint_mode<LAT, XLBH_F32, float, COLL>(p, s, call);
+        case XLBH_F16: return launch_adjoint_mode<LAT, XLBH_F16, float, COLL>(p, s, call);
+        case XLBH_BF16: return launch_adjoint_mode<LAT, XLBH_BF16, float, COLL>(p, s, call);
         case XLBH_F16_SHIFTED:
-          return launch_adjoint_mode<LAT, XLBH_F16_SHIFTED, float, COLL>(p, s, mode, flag, lam, pulled_in, own_out);
+          return launch_adjoint_mode<LAT, XLBH_F16_SHIFTED, float, COLL>(p, s, call);
         case XLBH_BF16_SHIFTED:
-          return launch_adjoint_mode<LAT, XLBH_BF16_SHIFTED, float, COLL>(p, s, mode, flag, lam, pulled_in, own_out);
+          return launch_adjoint_mode<LAT, XLBH_BF16_SHIFTED, float, COLL>(p, s, call);
       }
     } else if (compute == XLBH_COMPUTE_F64) {
       switch (store) {
-        case XLBH_F64: return launch_adjoint_mode<LAT, XLBH_F64, double, COLL>(p, s, mode, flag, lam, pulled_in, own_out);
-        case XLBH_F32: return launch_adjoint_mode<LAT, XLBH_F32, double, COLL>(p, s, mode, flag, lam, pulled_in, own_out);
+        case XLBH_F64: return launch_adjoint_mode<LAT, XLBH_F64, double, COLL>(p, s, call);
+        case XLBH_F32: return launch_adjoint_mode<LAT, XLBH_F32, double, COLL>(p, s, call);
       }
     }
     set_error("unsupported (store, compute) combination for the adjoint step");
     return 1;
   };
   // BEGIN / FLUSH do not depend on the collision
-  if (mode == ADJ_BEGIN || mode == ADJ_FLUSH || p.collision == XLBH_BGK)
+  if (call.mode == ADJ_BEGIN || call.mode == ADJ_FLUSH || p.collision == XLBH_BGK)
     return with_coll(std::integral_constant<int, XLBH_BGK>{});
   if (p.collision == XLBH_SMAGORINSKY_BGK) return with_coll(std::integral_constant<int, XLBH_SMAGORINSKY_BGK>{});
   if constexpr (LAT != XLBH_D3Q19) {
@@ -1125,11 +1139,8 @@ int adjoint_dispatch_lat(int store, int compute, const AdjParams& p, hipStream_t
   return 1;
 }
 
-int adjoint_dispatch_d2q9(int store, int compute, const AdjParams& p, hipStream_t s, int mode, uint8_t* flag, void* lam,
-                          int pulled_in, int own_out);
-int adjoint_dispatch_d3q19(int store, int compute, const AdjParams& p, hipStream_t s, int mode, uint8_t* flag, void* lam,
-                          int pulled_in, int own_out);
-int adjoint_dispatch_d3q27(int store, int compute, const AdjParams& p, hipStream_t s, int mode, uint8_t* flag, void* lam,
-                          int pulled_in, int own_out);
+int adjoint_dispatch_d2q9(int store, int compute, const AdjParams& p, hipStream_t s, const AdjCall& call);
+int adjoint_dispatch_d3q19(int store, int compute, const AdjParams& p, hipStream_t s, const AdjCall& call);
+int adjoint_dispatch_d3q27(int store, int compute, const AdjParams& p, hipStream_t s, const AdjCall& call);
 
 }  // namespace xlbh

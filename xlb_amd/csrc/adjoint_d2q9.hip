@@ -3,8 +3,7 @@
 #include "adjoint.hpp"
 
 namespace xlbh {
-int adjoint_dispatch_d2q9(int store, int compute, const AdjParams& p, hipStream_t s, int mode, uint8_t* flag, void* lam,
-                          int pulled_in, int own_out) {
-  return adjoint_dispatch_lat<XLBH_D2Q9>(store, compute, p, s, mode, flag, lam, pulled_in, own_out);
+int adjoint_dispatch_d2q9(int store, int compute, const AdjParams& p, hipStream_t s, const AdjCall& call) {
+  return adjoint_dispatch_lat<XLBH_D2Q9>(store, compute, p, s, call);
 }
 }  // namespace xlbh

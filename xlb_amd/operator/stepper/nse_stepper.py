@@ -386,15 +386,16 @@ class IncompressibleNavierStokesStepper(Stepper):
         return torch.empty(nbytes, dtype=torch.uint8, device=bc_mask.device)
 
     def adjoint_run(self, f_ckpt, states, lam_a, lam_b, bc_mask, missing_mask, omega, num_steps, timestep=0,
-                    grad_force=None, recompute=True, workspace=None, begin=True, end=True):
+                    grad_force=None, recompute=True, workspace=None, begin=True, end=True, one_mask=False):
         """Reverse sweep over one checkpoint segment below the ABI (xlbh_adjoint_run_known): recompute the
         ``num_steps - 1`` states after ``f_ckpt`` into ``states`` ((num_steps - 1, q, ...) in the
         store dtype), then apply the adjoint steps in reverse starting from lam_a = dL/df at the
         segment end.  Returns the buffer (lam_a or lam_b) that holds dL/df_ckpt.  With
         ``recompute=False`` the states are taken as recorded by ``record``.  A ``workspace`` (from
         ``adjoint_workspace``) selects the fused one-kernel reverse step; a sweep over several
-        segments shares it, with ``begin`` on its first call and ``end`` on its last.  Every
-        collision (BGK, KBC, SmagorinskyLESBGK)."""
+        segments shares it, with ``begin`` on its first call and ``end`` on its last, and
+        ``one_mask`` if they all have the same masks (faster).  Every collision (BGK, KBC,
+        SmagorinskyLESBGK)."""
         self._check_adjoint_supported()
         if self._has_solid:
             raise NotImplementedError("the adjoint step does not support solid (255) cells")
@@ -415,7 +416,7 @@ class IncompressibleNavierStokesStepper(Stepper):
             need = int(_lib.lib().xlbh_adjoint_workspace_bytes(self.lattice_id, self.compute_id, nx, ny, nz))
             if workspace.dtype != torch.uint8 or workspace.numel() < need or not workspace.is_contiguous():
                 raise ValueError(f"workspace must be a contiguous uint8 tensor of >= {need} bytes")
-            flags |= (_lib.ADJ_BEGIN if begin else 0) | (_lib.ADJ_END if end else 0)
+            flags |= (_lib.ADJ_BEGIN if begin else 0) | (_lib.ADJ_END if end else 0) | (_lib.ADJ_ONE_MASK if one_mask else 0)
         _lib.check(
             _lib.lib().xlbh_adjoint_run_known(
                 self.lattice_id, self._collision_id(), self.precision_policy.store_format, self.compute_id,
