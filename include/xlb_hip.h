@@ -209,8 +209,10 @@ int xlbh_run_known(int lattice, int collision, int store, int compute,
 
 /* n_steps >= 1 steps from f_start, which is only read, through the two buffers f_a and f_b (f_b is
  * not used by a single step); *in_b (host) tells where the newest populations are: f_a (0) or f_b
- * (1).  The other buffer's contents are unspecified.  `known` as in xlbh_run_known.  For callers that
- * keep f_start (a checkpoint) and would otherwise copy it before xlbh_run. */
+ * (1).  The other buffer's contents are unspecified.  `known` as in xlbh_run_known.  The result is that
+ * of xlbh_run on two copies of f_start (solid cells keep f_start's populations; with XLBH_MASK_SOLID in
+ * `known` the mask is searched for them).  For callers that keep f_start (a checkpoint) and would
+ * otherwise copy it before xlbh_run. */
 int xlbh_advance(int lattice, int collision, int store, int compute,
                  const void* f_start, void* f_a, void* f_b,
                  const uint8_t* bc_mask, const uint32_t* missing_bits,

@@ -110,6 +110,39 @@ static int validate_step(int lattice, int collision, int store, int compute, con
   return 0;
 }
 
+// Populations of the solid cells (id 255) from f into a and, if given, b: the steps leave them as they
+// find them in their output buffer.
+template <class R>
+__global__ __launch_bounds__(256) void k_copy_solid(const uint8_t* __restrict__ mask, const R* __restrict__ f, R* a,
+                                                    R* b, int q, uint64_t P, uint64_t N) {
+  const uint64_t stride = (uint64_t)gridDim.x * 256u;
+  for (uint64_t cell = (uint64_t)blockIdx.x * 256u + threadIdx.x; cell < N; cell += stride) {
+    if (mask[cell] != 255) continue;
+    for (int l = 0; l < q; ++l) {
+      const R v = f[l * P + cell];
+      a[l * P + cell] = v;
+      if (b) b[l * P + cell] = v;
+    }
+  }
+}
+
+static int copy_solid(int lattice, const StepCall& c, void* a, void* b) {
+  const uint64_t N = (uint64_t)c.nx * c.ny * c.nz;
+  const dim3 grid((unsigned)std::min<uint64_t>((N + 255) / 256, 65536));
+  auto go = [&](auto r) {
+    using R = decltype(r);
+    hipLaunchKernelGGL(k_copy_solid<R>, grid, dim3(256), 0, c.stream, c.bc_mask, static_cast<const R*>(c.f_in),
+                       static_cast<R*>(a), static_cast<R*>(b), lattice_q(lattice), c.plane, N);
+  };
+  switch (store_bytes(c.store)) {
+    case 8: go(uint64_t{}); break;
+    case 4: go(uint32_t{}); break;
+    default: go(uint16_t{});
+  }
+  XLBH_LAUNCH_CHECK();
+  return 0;
+}
+
 }  // namespace xlbh
 
 using namespace xlbh;
@@ -228,6 +261,8 @@ int xlbh_advance(int lattice, int collision, int store, int compute, const void*
   if (int e = resolve_plane(lattice, store, nx, ny, nz, plane, P)) return e;
   StepCall c{collision, store, compute, f_start, f_a, bc_mask, missing_bits, aux, bc_table,
              force_mode, force_uniform, force_field, nx, ny, nz, P, omega, collision_param, (hipStream_t)stream};
+  if (bc_mask && (known & XLBH_MASK_SOLID))
+    if (int e = copy_solid(lattice, c, f_a, n_steps > 1 ? f_b : nullptr)) return e;
   const Launcher go = plan_steps(lattice, c, known, n_steps);
   const int launches = go.launches(n_steps);
   for (int k = 0, t = 0; k < launches; ++k) {

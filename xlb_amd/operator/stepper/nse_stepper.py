@@ -452,7 +452,8 @@ class IncompressibleNavierStokesStepper(Stepper):
     def advance(self, f_start, f_a, f_b, bc_mask, missing_mask, omega, num_steps, timestep=0):
         """``num_steps`` steps from ``f_start``, which is only read, through the buffers ``f_a`` and
         ``f_b`` (xlbh_advance); returns (newest, other), the one of the two that holds the newest
-        populations first.  Needs no copy of a state that is kept, as ``run`` would."""
+        populations first: what ``run`` makes of two copies of ``f_start`` (solid cells keep its
+        populations), without the copies."""
         nx, ny, nz, plane, masks, force_mode, fu_ptr, keep, force_field = self._launch_args(f_start, f_a, bc_mask, missing_mask)
         ext, fmt = (nx, ny, nz), self.precision_policy.store_format
         common_plane([plane, expect_population(f_b, self.velocity_set.q, ext, "f_b", self.store_dtype, self.lattice_id, fmt)],
