@@ -117,23 +117,21 @@ class _Rollout(torch.autograd.Function):
         ckpts = {}
         # the state of the masks, and the checks of a step: the first checkpoint is encoded before one
         stepper._launch_args(a, None, bc_mask, missing_mask)
-        if stepper._has_solid:
-            # solid cells keep what the two buffers held: the buffers of a plain run, and copies
-            b = torch.empty_like(a)
-            for s in range(0, num_steps, every):
-                ckpts[s] = _Checkpoint(a.clone() if ckpt_mode == "store" else a, ckpt_mode, w, stepper)
-                a, b = stepper.run(a, b, bc_mask, missing_mask, omega, min(every, num_steps - s), timestep=s)
-        else:
-            # a checkpoint in the store dtype is the state itself, which the steps only read
+        if ckpt_mode == "store" and not stepper._has_solid:
+            # the checkpoint is the state itself, which the steps only read
             free = []
             for s in range(0, num_steps, every):
                 ckpts[s] = _Checkpoint(a, ckpt_mode, w, stepper)
                 b, c = (free.pop() if free else torch.empty_like(a) for _ in range(2))
-                new, other = stepper.advance(a, b, c, bc_mask, missing_mask, omega, min(every, num_steps - s), timestep=s)
+                a, other = stepper.advance(a, b, c, bc_mask, missing_mask, omega, min(every, num_steps - s), timestep=s)
                 free.append(other)
-                if ckpt_mode != "store":
-                    free.append(a)
-                a = new
+        else:
+            # an encoded checkpoint holds the state already, so two fields do; solid cells keep what
+            # the two buffers of a plain run held
+            b = torch.empty_like(a)
+            for s in range(0, num_steps, every):
+                ckpts[s] = _Checkpoint(a.clone() if ckpt_mode == "store" else a, ckpt_mode, w, stepper)
+                a, b = stepper.run(a, b, bc_mask, missing_mask, omega, min(every, num_steps - s), timestep=s)
         ctx.stepper = stepper
         ctx.masks = (bc_mask, missing_mask)
         ctx.omega = omega
