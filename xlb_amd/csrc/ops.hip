@@ -95,27 +95,34 @@ __device__ __forceinline__ C ld_pop_at(const typename Fmt<FMT>::raw* f, uint64_t
 // Moments: which = 0 rho+u, 1 rho, 2 u given rho, 3 Pi (macroscopic.py:39-55,
 // zero_moment.py:29-42, first_moment.py:40-56, second_moment.py:81-98).
 // ------------------------------------------------------------------------------------------
-// Bound by the populations' reads.  nt: they are read past the caches, so the velocity just written
-// stays in the memory-side cache for what reads it next: FP32 D3Q19 256^3 moments, vorticity and
-// Q-criterion 471 -> 430 us, 300x200x230 445 -> 409, FP64 128^3 134 -> 126.
-template <int LAT, int FMT, class C, class FR>
+// Bound by the populations' reads, taken one cell after another: rows do not matter here (but for the
+// segments of the block format), and tiles of rows idle lanes and split the cache lines that two rows
+// share (moments after a step, us: FP32 D3Q19 150x150x130 53 -> 49, FP16 40 -> 30).  NT: they are read
+// past the caches, so the velocity just written stays in the memory-side cache for what reads it next
+// (FP32 D3Q19 256^3: moments 265 -> 239, with vorticity and Q-criterion 478 -> 376; 300x200x230 253 ->
+// 223, 449 -> 345).
+template <int LAT, int FMT, class C, class FR, bool NT>
 __global__ __launch_bounds__(256) void k_moments(const typename Fmt<FMT>::raw* __restrict__ f, FR* rho,
-                                                 FR* u, FR* pi, int which, int nt, Sweep sw, uint32_t N, uint64_t P) {
+                                                 FR* u, FR* pi, int which, Sweep sw, uint32_t N, uint64_t P) {
   constexpr LatTables T = make_tables(LAT);
-  int x, y, z;
-  if (!sweep_cell(sw, x, y, z)) return;
-  const uint32_t cell = ((uint32_t)x * sw.ny + y) * sw.nz + z;
+  uint32_t cell = blockIdx.x * 256u + threadIdx.x;
   const int32_t* e = reinterpret_cast<const int32_t*>(reinterpret_cast<const char*>(f) + blk_exps_offset(T.q, P));
-  const int k = FMT == XLBH_I16_BLOCK ? e[blk_seg(sw, x, y, z)] : 0;
+  int k = 0;
+  if constexpr (FMT == XLBH_I16_BLOCK) {
+    int x, y, z;
+    if (!sweep_cell(sw, x, y, z)) return;
+    cell = ((uint32_t)x * sw.ny + y) * sw.nz + z;
+    k = e[blk_seg(sw, x, y, z)];
+  } else if (cell >= N) {
+    return;
+  }
   C ff[T.q];
-  if (FMT != XLBH_I16_BLOCK && nt != 0) {
-    asm volatile("; nt" ::: "memory");  // keeps the two branches' loads from being merged into plain ones
 #pragma unroll
-    for (int l = 0; l < T.q; ++l) ff[l] = ld_pop<FMT, C, true>(f + (size_t)l * P + cell, T.w[l]);
-    asm volatile("; nt" ::: "memory");
-  } else {
-#pragma unroll
-    for (int l = 0; l < T.q; ++l) ff[l] = ld_pop_at<LAT, FMT, C>(f, P, e, k, l, cell);
+  for (int l = 0; l < T.q; ++l) {
+    if constexpr (NT)
+      ff[l] = ld_pop<FMT, C, true>(f + (size_t)l * P + cell, T.w[l]);
+    else
+      ff[l] = ld_pop_at<LAT, FMT, C>(f, P, e, k, l, cell);
   }
   if (which == 3) {
 #pragma unroll
@@ -459,14 +466,27 @@ int xlbh_moments(int lattice, int store, int compute, int field, int which, cons
       using C = decltype(c);
       return with_field(field, [&](auto fr) -> int {
         using FR = decltype(fr);
-        // nt where the populations do not fit the memory-side cache (256 MB) and the velocity does.
-        // Smaller ones are still there when they are read again (FP32 128^3 62 -> 65 us with nt), a
-        // larger velocity does not stay (FP64 300x200x230 926 -> 945).
-        const uint64_t cache = 256ull << 20;
-        const int nt = (which == 0 || which == 2) && (uint64_t)Lat<LAT>::Q * N * sizeof(typename Fmt<FMT>::raw) > cache &&
-                       (uint64_t)Lat<LAT>::D * N * sizeof(FR) <= cache;
-        hipLaunchKernelGGL((k_moments<LAT, FMT, C, FR>), sweep_grid(sw), dim3(256), 0, s,
-                           (const typename Fmt<FMT>::raw*)f, (FR*)rho, (FR*)u, (FR*)pi, which, nt, sw, N, P);
+        // NT where the populations do not fit the memory-side cache (256 MB) and the velocity does.
+        // Smaller ones are still there when they are read again (FP32 D3Q19 128^3 33.5 -> 39.7 us with
+        // NT), a larger velocity does not stay.  Planes that start inside a cache line share it with
+        // the one before, and need more to make up for reading it twice (D3Q27 FP32 86x238x139, 293 MB:
+        // 62 -> 72; FP64 D3Q19, 412 MB: 97 -> 92).
+        const uint64_t cache = 256ull << 20, size = sizeof(typename Fmt<FMT>::raw);
+        const uint64_t least = P * size % 128 == 0 ? cache : cache + cache / 2;
+        const bool nt = (which == 0 || which == 2) && Lat<LAT>::Q * N * size > least && (uint64_t)Lat<LAT>::D * N * sizeof(FR) <= cache;
+        auto go = [&](auto streamed) {
+          const dim3 grid = FMT == XLBH_I16_BLOCK ? sweep_grid(sw) : dim3((N + 255u) / 256u);
+          hipLaunchKernelGGL((k_moments<LAT, FMT, C, FR, decltype(streamed)::value>), grid, dim3(256), 0, s,
+                             (const typename Fmt<FMT>::raw*)f, (FR*)rho, (FR*)u, (FR*)pi, which, sw, N, P);
+        };
+        if constexpr (FMT != XLBH_I16_BLOCK) {
+          if (nt) {
+            go(std::true_type{});
+            XLBH_LAUNCH_CHECK();
+            return 0;
+          }
+        }
+        go(std::false_type{});
         XLBH_LAUNCH_CHECK();
         return 0;
       });
