@@ -416,8 +416,14 @@ StepParams step_params(const StepCall& c) {
   p.plane = c.plane;
   // Non-temporal stores only where rows are whole 128-byte lines: of a line shared by two rows the
   // halves would go out one by one (D3Q19 FP32 101x83x77: 25.1 us per step, 19.9 without; 300x200x230
-  // 539 and 483; D3Q27 101x83x77 36.3 and 27.5; 256^3 the other way round, 428 and 443).
-  p.nt = (uint64_t)(c.nz > 1 ? c.nz : c.ny) * sizeof(typename Fmt<FMT>::raw) % 128 == 0;
+  // 539 and 483; D3Q27 101x83x77 36.3 and 27.5; 256^3 the other way round, 428 and 443).  A 2-D row shares
+  // one line in many, which the caches merge if they hold it for long enough: plain stores are the
+  // faster ones only for fields of 32 MB and more without boundary cells (FP32 1178x1555 periodic 31.2
+  // and 24.0; but FP64 911x177 7.5 and 9.1, FP32 1517x2323 channel 58.9 and 65.6).
+  using Raw = typename Fmt<FMT>::raw;
+  const bool lines = (uint64_t)(c.nz > 1 ? c.nz : c.ny) * sizeof(Raw) % 128 == 0;
+  const bool big = (uint64_t)Lat<LAT>::Q * p.N * sizeof(Raw) >= 32ull << 20;
+  p.nt = lines || (Lat<LAT>::D == 2 && (c.bc_mask || !big));
   p.per_xcd = 0;
   p.e_in = nullptr;
   p.e_out = nullptr;
