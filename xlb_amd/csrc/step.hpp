@@ -447,20 +447,21 @@ int launch_step_t(const StepCall& c) {
     if constexpr (Lat<LAT>::D == 3 && FMT != XLBH_I16_BLOCK) {
       // Rows that do not fill their tiles leave lanes idle (nz = 77: 40 %, 320: 38 %) and start in the
       // middle of cache lines; consecutive cells of the whole x-plane do not.  Grids of up to 3 M
-      // cells, whose planes the L2s and the memory-side cache still hold from the step before, go
-      // slab-wise over the XCDs.  us per step with tiles, flat, flat in slabs:
+      // cells (1.5 M in 8 bytes), whose planes the L2s and the memory-side cache still hold from the step
+      // before, go slab-wise over the XCDs.  us per step with tiles, flat, flat in slabs:
       //   D3Q19 FP32  40x40x40 5.0 5.0 4.3, 72x32x41 5.1 6.0 4.6, 101x83x77 19.9 18.6 16.5,
       //               100x100x320 70 67.2 68.1, 300x200x230 347 330 333, 360x360x300 1090 923 935
       //   D3Q19 FP16  72x32x41 4.8 4.8 4.1, 101x83x77 13.7 11.8 10.6, 64x60x600 35.5 33 29.3,
       //               200x160x200 128 91.5 98
-      //   D3Q19 FP64  72x32x41 7.9 8.5 6.4, 101x83x77 33.6 33.2 30.9
+      //   D3Q19 FP64  72x32x41 7.9 8.5 6.4, 101x83x77 33.6 33.2 30.9, 55x127x227 101 103 112
       //   D3Q27 FP32  72x32x41 6.3 8.1 5.6, 101x83x77 27.5 25.8 22.9, 200x160x200 321 260 266
+      //   D3Q27 FP64  140x96x180 260 215 285
       // Whole tiles keep the scalar row addresses (256^3 D3Q19 FP32: 428, flat 437); in slabs they gain
       // and lose by up to a fifth (48x48x64 6.8 and 5.6, D3Q27 FP64 120x60x256 150 and 174).
       if (!wide && (c.nz & ((1 << p.sw.lbz) - 1)) != 0) {
         const uint32_t per_plane = (uint32_t)(((uint64_t)c.ny * c.nz + 255) / 256), planes = (uint32_t)(p.x1 - p.x0);
         const dim3 grid(per_plane, planes);
-        if (p.N <= (3u << 20)) p.per_xcd = per_plane * planes / 8;
+        if (p.N <= (3u << 20) / (sizeof(typename Fmt<FMT>::raw) == 8 ? 2 : 1)) p.per_xcd = per_plane * planes / 8;
         if constexpr (w6)
           hipLaunchKernelGGL((k_step_w6<LAT, COLL, FMT, C, false, MS, true>), grid, dim3(256), lds, c.stream, p);
         else
