@@ -207,6 +207,12 @@ int xlbh_run_known(int lattice, int collision, int store, int compute,
                    int nx, int ny, int nz, int64_t plane, double omega, double collision_param, int timestep0,
                    int n_steps, uint32_t known, void* stream);
 
+/* The kernel launches xlbh_run_known (keep = 0) or xlbh_record_known (keep = 1) makes for n_steps steps
+ * of such a call, fewer than n_steps where one launch does several; has_mask tells whether it has a
+ * bc_mask.  -1 for invalid arguments.  No GPU is needed. */
+int xlbh_run_launches(int lattice, int collision, int store, int compute, int has_mask, int force_mode, int nx, int ny,
+                      int nz, int n_steps, uint32_t known, int keep);
+
 /* n_steps >= 1 steps from f_start, which is only read, through the two buffers f_a and f_b (f_b is
  * not used by a single step); *in_b (host) tells where the newest populations are: f_a (0) or f_b
  * (1).  The other buffer's contents are unspecified.  `known` as in xlbh_run_known.  The result is that

@@ -68,6 +68,7 @@ SIGNATURES = {
     "xlbh_run": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _dp, _vp, _i, _i, _i, _i64, _d, _d, _i, _i, _vp]),
     "xlbh_run_known": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _dp, _vp, _i, _i, _i, _i64, _d, _d, _i, _i,
                             _u32, _vp]),
+    "xlbh_run_launches": (_i, [_i, _i, _i, _i, _i, _i, _i, _i, _i, _i, _u32, _i]),
     "xlbh_advance": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _dp, _vp, _i, _i, _i, _i64, _d, _d, _i,
                           _i, _u32, _ip, _vp]),
     "xlbh_step_slab": (_i, [_i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _i, _dp, _vp, _i, _i, _i, _i64, _d, _d, _i, _i,

@@ -84,9 +84,9 @@ struct Launcher {
   }
 };
 
-static Launcher plan_steps(int lattice, const StepCall& c, uint32_t known, int n) {
+static Launcher plan_steps(int lattice, const StepCall& c, uint32_t known, int n, bool keep = false) {
   Launcher go;
-  if (n > 1 && steps_2d_apply(lattice, c, known)) go.per = steps_2d_best(c, n);
+  if (n > 1 && steps_2d_apply(lattice, c, known)) go.per = steps_2d_best(c, n, keep);
   if (n > 1 && plan_pair(lattice, c, known, go.tiles)) go.per = 2;
   return go;
 }
@@ -108,6 +108,20 @@ static int validate_step(int lattice, int collision, int store, int compute, con
   XLBH_REQUIRE(force_mode != XLBH_FORCE_UNIFORM || force_uniform, "uniform force needs 3 host doubles");
   XLBH_REQUIRE(force_mode != XLBH_FORCE_FIELD || force_field, "force field pointer is null");
   return 0;
+}
+
+// Launches of a run that is to leave both buffers as n one-step launches do.  Each launch writes the
+// buffer it does not read: as many launches as n in parity, the last of them of one step, leave the
+// newest state in the buffer n selects and the one before it in the other.
+static int run_launches(const Launcher& go, int n) {
+  const int launches = n > 0 ? 1 + go.launches(n - 1) : 0;
+  return launches + ((launches ^ n) & 1);
+}
+
+static Launcher plan_record(int lattice, const StepCall& c, uint32_t known, int n) {
+  // (Two 3-D steps per launch that keep the first one's state too save little: 256^3 434 us per step
+  // either way, 128^3 62 against 67 us.)
+  return lattice == XLBH_D2Q9 ? plan_steps(lattice, c, known, n, true) : Launcher();
 }
 
 // Populations of the solid cells (id 255) from f into a and, if given, b: the steps leave them as they
@@ -227,12 +241,8 @@ int xlbh_run_known(int lattice, int collision, int store, int compute, void* f_a
   if (int e = resolve_plane(lattice, store, nx, ny, nz, plane, P)) return e;
   StepCall c{collision, store, compute, f_a, f_b, bc_mask, missing_bits, aux, bc_table,
              force_mode, force_uniform, force_field, nx, ny, nz, P, omega, collision_param, (hipStream_t)stream};
-  // Each launch writes the buffer it does not read.  As many launches as n_steps in parity, the last
-  // of them of one step, leave both buffers as n_steps one-step launches do: the newest state in
-  // the buffer n_steps selects, the one before it in the other.
   const Launcher go = plan_steps(lattice, c, known, n_steps - 1);
-  int launches = n_steps > 0 ? 1 + go.launches(n_steps - 1) : 0;
-  launches += (launches ^ n_steps) & 1;
+  const int launches = run_launches(go, n_steps);
   for (int k = 0, t = 0; k < launches; ++k) {
     c.f_in = (k % 2 == 0) ? f_a : f_b;
     c.f_out = (k % 2 == 0) ? f_b : f_a;
@@ -304,10 +314,7 @@ int xlbh_record_known(int lattice, int collision, int store, int compute, const 
   const size_t field_bytes = (size_t)xlbh_population_bytes(lattice, store, nx, ny, nz, (int64_t)P);
   StepCall c{collision, store, compute, f_start, states, bc_mask, missing_bits, aux, bc_table,
              force_mode, force_uniform, force_field, nx, ny, nz, P, omega, collision_param, (hipStream_t)stream};
-  // (Two 3-D steps per launch that keep the first one's state too save little: 256^3 434 us per step
-  // either way, 128^3 62 against 67 us.)
-  Launcher go;
-  if (lattice == XLBH_D2Q9) go = plan_steps(lattice, c, known, n_states);
+  const Launcher go = plan_record(lattice, c, known, n_states);
   // A recording may start from one of the states it overwrites, which its first step reads: a launch
   // of several steps would write that state while other blocks still read it.
   const uintptr_t at = (uintptr_t)f_start, kept = (uintptr_t)states;
@@ -321,6 +328,25 @@ int xlbh_record_known(int lattice, int collision, int store, int compute, const 
     j += m;
   }
   return 0;
+}
+
+int xlbh_run_launches(int lattice, int collision, int store, int compute, int has_mask, int force_mode, int nx, int ny,
+                      int nz, int n_steps, uint32_t known, int keep) {
+  clear_error();
+  const void *f = &known, *g = &keep;  // stand-ins: only whether a pointer is null counts here
+  const double no_force[3] = {0.0, 0.0, 0.0};
+  const uint8_t* mask = has_mask ? static_cast<const uint8_t*>(f) : nullptr;
+  if (validate_step(lattice, collision, store, compute, f, g, mask, static_cast<const uint32_t*>(f),
+                    static_cast<const xlbh_bc_desc*>(f), force_mode, no_force, f, nx, ny, nz))
+    return -1;
+  if (n_steps < 0) {
+    set_error("n_steps must be >= 0");
+    return -1;
+  }
+  const StepCall c{collision, store, compute, f, const_cast<void*>(g), mask, nullptr, nullptr, nullptr,
+                   force_mode, no_force, f, nx, ny, nz, 0, 1.0, 0.0, nullptr};
+  if (keep) return plan_record(lattice, c, known, n_steps).launches(n_steps);
+  return run_launches(plan_steps(lattice, c, known, n_steps - 1), n_steps);
 }
 
 int xlbh_record(int lattice, int collision, int store, int compute, const void* f_start, void* states,

@@ -17,7 +17,6 @@
 // step, FP32 (FP64), before and after: channel with a force field 64x64 4.1 -> 1.9 (4.5 -> 2.4),
 // 512x256 5.2 -> 3.3 (6.3 -> 4.4), 1024x512 12.3 -> 8.3 (20.2 -> 15.3), 2048x2048 73 -> 46 (136 -> 97);
 // periodic 64x64 2.9 -> 0.9, 512x256 4.5 -> 2.7, 1024x512 10.3 -> 5.0, 2048x2048 62 -> 34.
-// Non-temporal stores: 512x256 channel 3.7 -> 3.3.
 #pragma once
 
 #include "step.hpp"
@@ -33,7 +32,8 @@ struct Steps2d {
   size_t state_bytes;  // when every state is kept: bytes from one to the next, else 0
 };
 
-template <int COLL, int FMT, class C, bool BCS>
+// BCS: there is a mask; NT: non-temporal stores.
+template <int COLL, int FMT, class C, bool BCS, bool NT>
 __global__ __launch_bounds__(kTile2d * kTile2d, sizeof(C) == 4 && COLL != XLBH_KBC ? 8 : 4) void k_steps_2d(StepParams p, Steps2d g) {
   constexpr int LAT = XLBH_D2Q9;
   constexpr LatTables T = make_tables(LAT);
@@ -138,7 +138,7 @@ __global__ __launch_bounds__(kTile2d * kTile2d, sizeof(C) == 4 && COLL != XLBH_K
       if (inner && (s == n || g.state_bytes != 0)) {
         R* out = reinterpret_cast<R*>(static_cast<char*>(p.f_out) + (g.state_bytes != 0 ? (s - 1) * g.state_bytes : 0));
 #pragma unroll
-        for (int l = 0; l < Q; ++l) st_pop<FMT, C>(out + l * p.plane + cell, f[l], T.w[l]);
+        for (int l = 0; l < Q; ++l) st_pop<FMT, C, NT>(out + l * p.plane + cell, f[l], T.w[l]);
       }
     }
     __syncthreads();
@@ -148,8 +148,8 @@ __global__ __launch_bounds__(kTile2d * kTile2d, sizeof(C) == 4 && COLL != XLBH_K
 // Whether several steps of a call can run as one launch.  `known`: what may occur in the mask
 // (XLBH_MASK_*, kind bits).
 bool steps_2d_apply(int lattice, const StepCall& c, uint32_t known);
-// Steps per launch that take the least time for a run of `n` steps.
-int steps_2d_best(const StepCall& c, int n);
+// Steps per launch that take the least time for a run of `n` steps (1: k_step); keep: every state is kept.
+int steps_2d_best(const StepCall& c, int n, bool keep);
 // `steps` steps from c.f_in to c.f_out; with state_bytes != 0 the state after step s goes to
 // c.f_out + (s - 1) * state_bytes.
 int launch_steps_2d(const StepCall& c, int steps, size_t state_bytes);
