@@ -113,7 +113,7 @@ typedef struct xlbh_bc_desc {
 /* Message of the last failed call on this thread ("" if none). */
 const char* xlbh_last_error(void);
 
-/* ABI version of this header (incremented on incompatible change). */
+/* ABI version of this header (incremented when entries are added or changed). */
 int xlbh_abi_version(void);
 
 /* Plane stride (elements) this library recommends for population fields of the given grid and

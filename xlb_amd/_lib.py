@@ -35,7 +35,7 @@ FORCE_NONE, FORCE_UNIFORM, FORCE_FIELD = 0, 1, 2
 ADJ_RECOMPUTE, ADJ_BEGIN, ADJ_END, ADJ_ONE_MASK = 1, 2, 4, 8
 MASK_SOLID, MASK_FAR_OUTFLOW = 1 << 30, 1 << 29
 
-ABI_VERSION = 4
+ABI_VERSION = 5
 
 
 class BcDesc(ctypes.Structure):
@@ -120,13 +120,13 @@ def lib():
             "(or __graft_entry__.build()). There is no fallback implementation."
         )
     L = ctypes.CDLL(LIB_PATH)
+    v = L.xlbh_abi_version()  # before the entries are looked up: an older library lacks some
+    if v != ABI_VERSION:
+        raise RuntimeError(f"libxlbhip.so ABI version {v} != expected {ABI_VERSION}; rebuild it")
     for name, (res, args) in SIGNATURES.items():
         fn = getattr(L, name)
         fn.restype = res
         fn.argtypes = args
-    v = L.xlbh_abi_version()
-    if v != ABI_VERSION:
-        raise RuntimeError(f"libxlbhip.so ABI version {v} != expected {ABI_VERSION}; rebuild it")
     _LIB = L
     return L
 

@@ -165,7 +165,7 @@ extern "C" {
 
 const char* xlbh_last_error(void) { return g_last_error.c_str(); }
 
-int xlbh_abi_version(void) { return 4; }
+int xlbh_abi_version(void) { return 5; }
 
 int64_t xlbh_plane_stride(int lattice, int store, int nx, int ny, int nz) {
   clear_error();
