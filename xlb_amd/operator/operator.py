@@ -4,12 +4,14 @@
 registered for (class name, backend) is tried with the call's arguments; if none binds and runs,
 a generic ``Exception`` carrying the last error and its traceback is raised
 (operator.py:54-74).  Signatures are computed once at registration, the implementations of a class
-are looked up once, and a call is bound to a signature only to report why it failed (a call that
-does not bind raises TypeError before the implementation runs).
+are looked up once, and a call of a plain function is bound to its signature only to report why it
+failed (a call that does not bind raises TypeError before the function runs; a decorated one may take
+more than its signature says).
 """
 
 import inspect
 import traceback
+import types
 
 from xlb_amd import _lib
 from xlb_amd.compute_backend import ComputeBackend
@@ -20,6 +22,7 @@ from xlb_amd.precision_policy import Precision
 class Operator:
     _backends = {}
     _signatures = {}
+    _bind_first = set()  # implementations whose signature is not their own: calls are bound to it first
     _candidates = {}  # (class, backend) of past calls -> its implementations; cleared by a registration
 
     def __init__(self, velocity_set=None, precision_policy=None, compute_backend=None):
@@ -39,6 +42,8 @@ class Operator:
             key = (subclass_name, backend_name, str(signature))
             cls._backends[key] = func
             cls._signatures[key] = signature
+            own = isinstance(func, types.FunctionType) and not (hasattr(func, "__wrapped__") or hasattr(func, "__signature__"))
+            (cls._bind_first.discard if own else cls._bind_first.add)(key)
             Operator._candidates.clear()
             return func
 
@@ -61,6 +66,8 @@ class Operator:
         error, traceback_str, key = None, "", None
         for key, backend_method in self._implementations():
             try:
+                if key in self._bind_first:
+                    self._signatures[key].bind(self, *args, **kwargs)
                 result = backend_method(self, *args, **kwargs)
                 if callback and callable(callback):
                     callback(result if result is not None else (args, kwargs))
