@@ -47,3 +47,29 @@ def test_a_decorated_implementation_takes_what_its_signature_says(how):
     with pytest.raises(Exception, match="too many positional"):
         cls()(2, 3, 4)
     assert len(ran) == 1
+
+
+def test_an_implementation_registered_during_a_look_up_is_found_by_the_next_call():
+    """As when another thread imports the module that registers it."""
+    cls = _operator("AddUp")
+
+    def register(func):
+        func.__qualname__ = "AddUp.implementation"
+        cls.register_backend(BACKEND)(func)
+
+    class Table(dict):
+        late = None
+
+        def items(self):
+            seen = list(super().items())
+            if self.late is not None:
+                late, self.late = self.late, None
+                register(late)
+            return seen
+
+    cls._backends, cls._signatures = Table(), {}
+    register(lambda self, a: a)
+    cls._backends.late = lambda self, a, b: a + b
+    with pytest.raises(Exception):
+        cls()(1, 2)
+    assert cls()(1, 2) == 3

@@ -23,7 +23,7 @@ class Operator:
     _backends = {}
     _signatures = {}
     _bind_first = set()  # implementations whose signature is not their own: calls are bound to it first
-    _candidates = {}  # (class, backend) of past calls -> its implementations; cleared by a registration
+    _candidates = {}  # (class, backend) of past calls -> its implementations, since the last registration
 
     def __init__(self, velocity_set=None, precision_policy=None, compute_backend=None):
         self.velocity_set = velocity_set or DefaultConfig.velocity_set
@@ -44,14 +44,15 @@ class Operator:
             cls._signatures[key] = signature
             own = isinstance(func, types.FunctionType) and not (hasattr(func, "__wrapped__") or hasattr(func, "__signature__"))
             (cls._bind_first.discard if own else cls._bind_first.add)(key)
-            Operator._candidates.clear()
+            Operator._candidates = {}  # a new one: a look-up under way in another thread keeps to the old
             return func
 
         return decorator
 
     def _implementations(self):
         """[(key, method)] of the first class in the MRO with implementations for the backend."""
-        cached = self._candidates.get((type(self), self.compute_backend.name))
+        known = Operator._candidates
+        cached = known.get((type(self), self.compute_backend.name))
         if cached is not None:
             return cached
         found = []
@@ -59,7 +60,7 @@ class Operator:
             found = [(k, m) for k, m in self._backends.items() if k[0] == klass.__name__ and k[1] == self.compute_backend]
             if found:
                 break
-        self._candidates[type(self), self.compute_backend.name] = found
+        known[type(self), self.compute_backend.name] = found
         return found
 
     def __call__(self, *args, callback=None, **kwargs):
