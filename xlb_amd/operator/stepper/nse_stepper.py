@@ -33,6 +33,21 @@ from xlb_amd.operator.operator import Operator, common_plane, expect_field, expe
 from xlb_amd.operator.stream import Stream
 
 
+def far_outflow_patterns(c):
+    """(2^q,) bool: for each set of missing directions, whether an extrapolation outflow with them
+    reads a source x - c_l - n more than one cell away along an axis; its normal n and its missing l
+    are taken as the step kernel does (helper_functions_bc.py:75-86)."""
+    c = np.asarray(c)
+    bits = np.arange(1 << c.shape[1])
+    far, normal_found = np.zeros(bits.size, dtype=bool), np.zeros(bits.size, dtype=bool)
+    for m in (l for l in range(c.shape[1]) if np.abs(c[:, l]).sum() == 1):
+        beyond = sum(1 << l for l in range(c.shape[1]) if np.abs(c[:, l] - c[:, m]).max() > 1)
+        first = (bits >> m & 1 == 1) & ~normal_found
+        far |= first & (bits & beyond != 0)
+        normal_found |= first
+    return far
+
+
 class Stepper(Operator):
     """Base of steppers (stepper.py:6-34)."""
 
@@ -82,6 +97,7 @@ class IncompressibleNavierStokesStepper(Stepper):
         self._has_bc_cells = True
         self._has_solid = False
         self._mask_holds = 0
+        self._far_patterns = None
         self._bc_cells = None
         self._mask_ref = None
 
@@ -164,15 +180,20 @@ class IncompressibleNavierStokesStepper(Stepper):
         expect_field(missing_mask, self.velocity_set.q, ext, "missing_mask", torch.bool)
         self._bits = packed_missing(missing_mask, self.lattice_id)
         self._table = self._build_table(bc_mask.device)
-        self._has_bc_cells = bool(bc_mask.any().item())
-        self._has_solid = self._has_bc_cells and bool((bc_mask == 255).any().item())
         # what the mask may hold (xlbh_run_known): the kinds of this stepper's boundary conditions,
-        # ids of others (their table entry is empty: kind NONE) and solid cells
-        self._mask_holds = 1 << _lib.BC_NONE | (_lib.MASK_SOLID if self._has_solid else 0)
+        # ids of others (their table entry is empty: kind NONE), solid cells and far outflows; what has
+        # to be looked up comes back in one copy
+        holds = 1 << _lib.BC_NONE
+        found = [bc_mask.any(), (bc_mask == 255).any()]
         for bc in self.boundary_conditions:
-            self._mask_holds |= 1 << bc.kind
-            if self._has_bc_cells and bc.kind == _lib.BC_EXTRAPOLATION_OUTFLOW and self._far_outflow(bc.id, bc_mask):
-                self._mask_holds |= _lib.MASK_FAR_OUTFLOW
+            holds |= 1 << bc.kind
+            if bc.kind == _lib.BC_EXTRAPOLATION_OUTFLOW:
+                if self.velocity_set.d == 2:
+                    found.append(self._far_outflow(bc.id, bc_mask))
+                else:  # not looked up: no 3-D run depends on it
+                    holds |= _lib.MASK_FAR_OUTFLOW
+        self._has_bc_cells, self._has_solid, *far = map(bool, torch.stack(found).tolist())
+        self._mask_holds = holds | (_lib.MASK_SOLID if self._has_solid else 0) | (_lib.MASK_FAR_OUTFLOW if any(far) else 0)
         self._bc_cells = None
         nx, ny, nz = field_extents(bc_mask)
         aux_bcs = [bc for bc in self.boundary_conditions if bc.needs_aux_init]
@@ -185,17 +206,11 @@ class IncompressibleNavierStokesStepper(Stepper):
         self._state_key = self._mask_key(bc_mask, missing_mask)
 
     def _far_outflow(self, bc_id, bc_mask):
-        """True if a cell of the extrapolation outflow ``bc_id`` reads a source x - c_l - n more than
-        one cell away along an axis (its normal n and its missing directions l taken as the step
-        kernel does, helper_functions_bc.py:75-86)."""
-        c = np.asarray(self.velocity_set.c)
-        main = [l for l in range(self.velocity_set.q) if np.abs(c[:, l]).sum() == 1]
-        for bits in torch.unique(self._bits[bc_mask.view(-1) == int(bc_id)]).tolist():
-            missing = [l for l in range(self.velocity_set.q) if bits >> l & 1]
-            normal = next((-c[:, l] for l in main if l in missing), np.zeros(len(c), dtype=c.dtype))
-            if any(np.abs(c[:, l] + normal).max() > 1 for l in missing):
-                return True
-        return False
+        """True (on the device) if a cell of the extrapolation outflow ``bc_id`` reads a source
+        x - c_l - n more than one cell away along an axis."""
+        if self._far_patterns is None or self._far_patterns.device != bc_mask.device:
+            self._far_patterns = torch.from_numpy(far_outflow_patterns(np.asarray(self.velocity_set.c))).to(bc_mask.device)
+        return (self._far_patterns.index_select(0, self._bits) & (bc_mask.view(-1) == int(bc_id))).any()
 
     def _force_args(self):
         col = self.collision
