@@ -41,3 +41,28 @@ def test_deriving_it_waits_for_the_gpu_twice_at_most(lattice, shape, corners):
     bm[0, 5, 6] = 255
     st._sync_state(bm, mm)
     assert st._has_solid is True and st._mask_holds & _lib.MASK_SOLID
+
+
+def test_a_new_missing_mask_in_the_place_of_a_freed_one():
+    """A tensor that takes the id, the memory and the version of one that was freed is another tensor."""
+    BC = xa.operator.boundary_condition
+    policy = xa.PrecisionPolicy.FP32FP32
+    vs = xa.velocity_set.D2Q9(policy, xa.ComputeBackend.MI355X)
+    xa.init(velocity_set=vs, default_backend=xa.ComputeBackend.MI355X, default_precision_policy=policy)
+    grid = xa.grid.grid_factory((40, 24), compute_backend=xa.ComputeBackend.MI355X)
+    bc = BC.HalfwayBounceBackBC(indices=grid.bounding_box_indices(remove_edges=True)["bottom"])
+    st = xa.operator.stepper.IncompressibleNavierStokesStepper(grid, [bc])
+    f_0, f_1, bm, mm = st.prepare_fields()
+    masks = [mm.cpu(), torch.zeros_like(mm).cpu()]
+    taken = set()
+    for i in range(20):
+        want = masks[i % 2]
+        missing = want.cuda()
+        place = (id(missing), missing.data_ptr(), missing._version)
+        again = place in taken
+        taken.add(place)
+        st(f_0, f_1, bm, missing, 1.2, 0)
+        bits = sum((want[l].reshape(-1).int() << l) for l in range(9))
+        assert torch.equal(st._bits.cpu(), bits), (i, again)
+        del missing
+    assert again  # it did happen here

@@ -13,6 +13,7 @@ table of prescribed values.  ``run`` moves the caller's step/swap loop below the
 """
 
 import ctypes
+import weakref
 
 import numpy as np
 import torch
@@ -100,6 +101,7 @@ class IncompressibleNavierStokesStepper(Stepper):
         self._far_patterns = None
         self._bc_cells = None
         self._mask_ref = None
+        self._missing_ref = None
 
     # ------------------------------------------------------------------ fields
     def prepare_fields(self, initializer=None):
@@ -172,7 +174,7 @@ class IncompressibleNavierStokesStepper(Stepper):
 
     def _sync_state(self, bc_mask, missing_mask):
         key = self._mask_key(bc_mask, missing_mask)
-        if key == self._state_key:
+        if key == self._state_key and self._missing_ref() is missing_mask:  # (ids are used again)
             return
         _lib.require_cuda(bc_mask, missing_mask)
         ext = field_extents(bc_mask)
@@ -203,6 +205,7 @@ class IncompressibleNavierStokesStepper(Stepper):
             for bc in aux_bcs:
                 bc.aux_data_init(None, None, bc_mask, missing_mask, aux=self._aux)
         self._mask_ref = bc_mask
+        self._missing_ref = weakref.ref(missing_mask)
         self._state_key = self._mask_key(bc_mask, missing_mask)
 
     def _far_outflow(self, bc_id, bc_mask):
