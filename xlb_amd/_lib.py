@@ -153,7 +153,8 @@ def stream_of(t=None):
     on a GPU has none (its pointer must not reach a kernel)."""
     if t is None:
         return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
-    require_cuda(t)
+    if not t.is_cuda:
+        require_cuda(t)
     return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 

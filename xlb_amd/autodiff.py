@@ -24,6 +24,7 @@ import torch
 
 from xlb_amd import _lib
 from xlb_amd.operator.collision import ForcedCollision
+from xlb_amd.operator.operator import expect_population, field_extents
 
 
 def equilibrium_torch(rho, u, velocity_set):
@@ -115,8 +116,10 @@ class _Rollout(torch.autograd.Function):
         # a private copy: the first checkpoint is kept while the caller may change f0
         a = f0.detach().to(stepper.store_dtype, copy=True, memory_format=torch.contiguous_format)
         ckpts = {}
-        # the state of the masks, and the checks of a step: the first checkpoint is encoded before one
-        stepper._launch_args(a, None, bc_mask, missing_mask)
+        # the checks of a step, before the first checkpoint is encoded
+        expect_population(a, stepper.velocity_set.q, field_extents(bc_mask), "f0", stepper.store_dtype, stepper.lattice_id,
+                          stepper.precision_policy.store_format)
+        stepper._sync_state(bc_mask, missing_mask)
         if ckpt_mode == "store" and not stepper._has_solid:
             # the checkpoint is the state itself, which the steps only read
             free = []

@@ -50,14 +50,16 @@ class Operator:
         return decorator
 
     def _implementations(self):
-        """[(key, method)] of the first class in the MRO with implementations for the backend."""
+        """[(key, method, signature to bind first or None)] of the first class in the MRO with
+        implementations for the backend."""
         known = Operator._candidates
         cached = known.get((type(self), self.compute_backend.name))
         if cached is not None:
             return cached
         found = []
         for klass in type(self).__mro__:
-            found = [(k, m) for k, m in self._backends.items() if k[0] == klass.__name__ and k[1] == self.compute_backend]
+            found = [(k, m, self._signatures[k] if k in self._bind_first else None) for k, m in self._backends.items()
+                     if k[0] == klass.__name__ and k[1] == self.compute_backend]
             if found:
                 break
         known[type(self), self.compute_backend.name] = found
@@ -65,10 +67,10 @@ class Operator:
 
     def __call__(self, *args, callback=None, **kwargs):
         error, traceback_str, key = None, "", None
-        for key, backend_method in self._implementations():
+        for key, backend_method, signature in self._implementations():
             try:
-                if key in self._bind_first:
-                    self._signatures[key].bind(self, *args, **kwargs)
+                if signature is not None:
+                    signature.bind(self, *args, **kwargs)
                 result = backend_method(self, *args, **kwargs)
                 if callback and callable(callback):
                     callback(result if result is not None else (args, kwargs))
