@@ -80,7 +80,7 @@ struct Launcher {
   int share(int n, int left) const { return (n + left - 1) / left; }
   int operator()(int lattice, const StepCall& c, int steps, size_t state_bytes = 0) const {
     if (steps == 1) return dispatch_step(lattice, c);
-    return lattice == XLBH_D2Q9 ? launch_steps_2d(c, steps, state_bytes) : launch_pair(lattice, c, tiles);
+    return lattice == XLBH_D2Q9 ? launch_steps_2d(c, steps, state_bytes) : launch_pair(c, tiles);
   }
 };
 

@@ -312,6 +312,6 @@ constexpr int kPairRowsF32 = 15, kPairRowsF64 = 7;
 // Whether two steps of a call can run as one launch, and its tiles (g.blocks > 0).  `known`: what
 // may occur in the mask (XLBH_MASK_*, XLBH_KIND bits).
 bool plan_pair(int lattice, const StepCall& c, uint32_t known, PairTiles& g);
-int launch_pair(int lattice, const StepCall& c, const PairTiles& g);
+int launch_pair(const StepCall& c, const PairTiles& g);
 
 }  // namespace xlbh

@@ -18,8 +18,7 @@ bool plan_pair(int lattice, const StepCall& c, uint32_t known, PairTiles& g) {
   return g.blocks > 0;
 }
 
-int launch_pair(int lattice, const StepCall& c, const PairTiles& g) {
-  (void)lattice;
+int launch_pair(const StepCall& c, const PairTiles& g) {
   constexpr int L = XLBH_D3Q19, S = XLBH_SMAGORINSKY_BGK;
   if (c.compute == XLBH_COMPUTE_F64)
     return c.collision == S ? launch_pair_t<L, S, XLBH_F64, double, kPairRowsF64>(c, g)

@@ -109,11 +109,9 @@ struct PullOffsets {
 // Everything after the pull for one cell with boundary id `id` (!= 255), in place on the
 // post-stream populations f: streaming-step BC, collision (+ force), collision-step BC and the
 // extrapolation-outflow update (nse_stepper.py:360-378).
-// `fin` reads stored populations other than the pulls: fin.own(l, ...) the cell's own pre-stream
-// population l, fin.at(l, ...) another cell's.
-template <int LAT, int COLL, int FMT, class C, class O, class In>
+template <int LAT, int COLL, int FMT, class C, class O>
 __device__ __forceinline__ void cell_update(C* f, int id, O cell, int x, int y, int z, const StepParams& p,
-                                            const In& fin) {
+                                            const PopIn<FMT, C, O>& fin) {
   constexpr LatTables T = make_tables(LAT);
   constexpr int Q = T.q;
   const int nx = p.sw.nx, ny = p.sw.ny, nz = p.sw.nz;
