@@ -3,8 +3,8 @@
 Headline workload (the reference's own benchmark, examples/performance/mlups_3d.py:45-90, at
 edge 256): D3Q19 BGK lid-driven cavity 256^3, rho = 1 / u = 0 equilibrium start, lid
 EquilibriumBC(rho=1, u=(0.02, 0, 0)) on the top face without edges, FullwayBounceBackBC on the
-other five full faces, omega = 1.0.  One step = one fused stream-collide-BC pass over the grid;
-the timed loop runs K steps with the buffer swap below the C ABI (xlbh_run), all inputs resident
+other five full faces, omega = 1.0.  One step = one fused stream-collide-BC update of the grid;
+the timed loop runs K steps with the buffer swap below the C ABI (xlbh_run_known), all inputs resident
 in HBM.  value = MLUPS = 256^3 K / t / 1e6 with the FP32/FP32 policy.
 
 Also reported on the same line:
@@ -26,20 +26,22 @@ Also reported on the same line:
 * slab -- one GPU's share of an x-sharded run: the 256^3 periodic D3Q19 BGK FP32 data as a slab
   of 256 planes plus two ghost planes, stepped with xlbh_step_slab at dense and at the library's
   recommended plane stride, beside the whole-domain step; edge planes, interior and ghost fill.
-roofline.achieved = algorithmic bytes per launch (2 Q S_store per cell) / average kernel duration
-from HIP events on the launch stream; roofline.traffic = FETCH_SIZE + WRITE_SIZE per launch from
-rocprofv3 (profiles/traffic_step_d3q19_cavity256.json, written by --summarize-pmc).
+roofline.achieved = algorithmic bytes (2 Q S_store per cell for every launch, xlbh_run_launches: a launch
+of the FP32 run does two steps with the state in between on chip) / time from HIP events on the launch
+stream; roofline.traffic = FETCH_SIZE + WRITE_SIZE per launch of the kernel named from rocprofv3
+(profiles/traffic_step_pair_d3q19_cavity256.json, written by --summarize-pmc).
 cpu_baseline = the C++/OpenMP oracle (the parity reference of the tests, a restatement of the
 reference algorithm) timed on a bounded number of steps of the headline workload on the host cores.
 
 Usage:
   python bench.py [--gpus 1] [--steps K] [--warmup W] [--size 256] [--no-cpu] [--quick]
   python bench.py --profile [--steps K]        # headline kernel + a 1 GiB copy, for rocprofv3
-  python bench.py --summarize-pmc FETCH.csv WRITE.csv   # -> profiles/traffic_step_d3q19_cavity256.json
+  python bench.py --summarize-pmc FETCH.csv WRITE.csv   # -> profiles/traffic_step*_d3q19_cavity256.json
 """
 
 import argparse
 import csv
+import gc
 import json
 import re
 import os
@@ -54,7 +56,7 @@ sys.path.insert(0, ROOT)
 METRIC = "MLUPS & % HBM roofline, D3Q19 BGK 256³ (FP32 vs FP16-store); adjoint/fwd time"
 HBM_PEAK_GBS = 8000.0
 COPY_CALIBRATION_BYTES = 1 << 30
-TRAFFIC_JSON = os.path.join(ROOT, "profiles", "traffic_step_d3q19_cavity{n}.json")
+TRAFFIC_JSON = os.path.join(ROOT, "profiles", "traffic_{kernel}_d3q19_cavity{n}.json")
 
 
 def log(msg):
@@ -71,6 +73,7 @@ def time_run(torch, wl, steps, warmup):
     st = wl.stepper
     f0, f1 = st.run(wl.f_0, wl.f_1, wl.bc_mask, wl.missing_mask, wl.omega, warmup)
     torch.cuda.synchronize()
+    gc.collect()  # a full collection (50 ms with torch's objects) would otherwise fall anywhere, also below
     stream = torch.cuda.current_stream()
     ev0, ev1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     t0 = time.perf_counter()
@@ -80,6 +83,28 @@ def time_run(torch, wl, steps, warmup):
     torch.cuda.synchronize()
     wall = time.perf_counter() - t0
     return wall, ev0.elapsed_time(ev1) / 1e3, f0, f1
+
+
+def launches_of(wl, steps):
+    """Kernel launches of ``stepper.run`` over ``steps`` steps of a workload (xlbh_run_launches)."""
+    from xlb_amd import _lib
+
+    st = wl.stepper
+    got = _lib.lib().xlbh_run_launches(
+        st.lattice_id, st._collision_id(), st.precision_policy.store_format, st.compute_id, int(st._has_bc_cells),
+        st._force_args()[0], *wl.f_0.shape[1:], steps, st._mask_holds, 0)
+    if got < 0:
+        raise RuntimeError("xlbh_run_launches refused the workload")
+    return got
+
+
+def moved(wl, f, steps, seconds, torch):
+    """Algorithmic bytes per cell and step of a run (each launch reads and writes every population once)
+    and the rate they were moved at."""
+    launches = launches_of(wl, steps)
+    bytes_per_lu = 2 * wl.stepper.velocity_set.q * store_bytes(torch, f) * launches / steps
+    return dict(launches=launches, steps_per_launch=steps / launches, bytes_per_lu=bytes_per_lu,
+                achieved_gbs=bytes_per_lu * f[0].numel() * steps / seconds / 1e9)
 
 
 def headline_leg(xa, torch, policy, n, steps, warmup, python_loop=True):
@@ -102,9 +127,7 @@ def headline_leg(xa, torch, policy, n, steps, warmup, python_loop=True):
         torch.cuda.synchronize()
         res["mlups_python_loop"] = cells * py_steps / (time.perf_counter() - t1) / 1e6
     res["finite"] = bool(torch.isfinite(f0.float()).all().item())
-    bpl = 2 * wl.stepper.velocity_set.q * store_bytes(torch, f0)
-    kernel_s = ev_s / steps
-    res.update(bytes_per_lu=bpl, kernel_ms=kernel_s * 1e3, achieved_gbs=bpl * cells / kernel_s / 1e9)
+    res.update(kernel_ms=ev_s / steps * 1e3, **moved(wl, f0, steps, ev_s, torch))
     del wl, f0, f1
     torch.cuda.empty_cache()
     return res
@@ -416,7 +439,7 @@ def les_cavity_leg(xa, torch, n, steps, warmup):
     cells = n**3
     res = dict(workload=f"D3Q19 SmagorinskyLESBGK (Cs 0.17) lid-driven cavity {n}^3, lid u = 0.06, tau = 0.501, "
                         f"FP32, {steps} steps", mlups=cells * steps / wall / 1e6, kernel_ms=ev_s / steps * 1e3,
-               achieved_gbs=152 * cells / (ev_s / steps) / 1e9)
+               **moved(wl, f0, steps, ev_s, torch))
     res["frac"] = res["achieved_gbs"] / HBM_PEAK_GBS
     res["finite"] = bool(torch.isfinite(f0).all().item())
     g = wl.stepper.grid
@@ -446,14 +469,14 @@ def les_cavity_leg(xa, torch, n, steps, warmup):
 
 
 def periodic_leg(xa, torch, n, steps, warmup):
-    """The pure step kernel: D3Q19 BGK FP32 periodic box without boundary conditions."""
+    """The pure step: D3Q19 BGK FP32 periodic box without boundary conditions."""
     from xlb_amd.workloads import periodic_box_3d
 
     wl = periodic_box_3d(n, xa.PrecisionPolicy.FP32FP32)
     wall, ev_s, f0, f1 = time_run(torch, wl, steps, warmup)
     cells = n**3
     res = dict(workload=f"D3Q19 BGK FP32 periodic {n}^3, no boundary conditions", mlups=cells * steps / wall / 1e6,
-               kernel_ms=ev_s / steps * 1e3, achieved_gbs=152 * cells / (ev_s / steps) / 1e9)
+               kernel_ms=ev_s / steps * 1e3, **moved(wl, f0, steps, ev_s, torch))
     res["frac"] = res["achieved_gbs"] / HBM_PEAK_GBS
     del wl, f0, f1
     torch.cuda.empty_cache()
@@ -675,8 +698,8 @@ def cpu_leg(n, budget_s=12.0, max_steps=40):
                 sample=f"{steps} steps of the {n}^3 D3Q19 BGK cavity (FP32) after 2 warm-up steps, C++/OpenMP oracle")
 
 
-def load_traffic(n):
-    path = TRAFFIC_JSON.format(n=n)
+def load_traffic(n, kernel):
+    path = TRAFFIC_JSON.format(kernel=kernel, n=n)
     if os.path.exists(path):
         with open(path) as fh:
             return json.load(fh).get("bytes_per_launch")
@@ -711,9 +734,10 @@ def _read_pmc(path, counter):
 def summarize_pmc(fetch_csv, write_csv, n):
     """FETCH_SIZE / WRITE_SIZE (KiB per dispatch) of each step kernel profiled, each scaled by what
     the same counter reads for the 1 GiB calibration copy (the first three copy dispatches of the
-    profiled process, issued by ``profile_pass`` before anything else is copied).  The FP32 step
-    kernel's figures go to profiles/traffic_step_d3q19_cavity{n}.json (the headline line's
-    ``traffic``); a 16-bit kernel's to profiles/traffic_step16_<store>_d3q19_cavity{n}.json."""
+    profiled process, issued by ``profile_pass`` before anything else is copied).  The FP32 kernels'
+    figures go to profiles/traffic_step_pair_d3q19_cavity{n}.json (two steps per launch: the headline
+    line's ``traffic``) and traffic_step_d3q19_cavity{n}.json (single steps); a 16-bit kernel's to
+    profiles/traffic_step16_<store>_d3q19_cavity{n}.json."""
     fetch, write = _read_pmc(fetch_csv, "FETCH_SIZE"), _read_pmc(write_csv, "WRITE_SIZE")
 
     def calib(rows):
@@ -743,8 +767,8 @@ def summarize_pmc(fetch_csv, write_csv, n):
                    fetch_bytes=step_fetch * f_scale * 1024.0, write_bytes=step_write * w_scale * 1024.0,
                    bytes_per_launch=traffic, algorithmic_bytes_per_launch=algorithmic,
                    traffic_over_algorithmic=traffic / algorithmic)
-        path = TRAFFIC_JSON.format(n=n) if store == 0 else os.path.join(
-            os.path.dirname(TRAFFIC_JSON), f"traffic_step16_{store_names[store]}_d3q19_cavity{n}.json")
+        short = ("step_pair" if "k_step_pair" in kernel else "step") if store == 0 else f"step16_{store_names[store]}"
+        path = TRAFFIC_JSON.format(kernel=short, n=n)
         with open(path, "w") as fh:
             json.dump(out, fh, indent=1)
         results[kernel] = out
@@ -856,6 +880,7 @@ def main():
         cpu = cpu_leg(n)
         log(f"bench: cpu {cpu['value']:.1f} MLUPS on {cpu['cores']} threads")
 
+    paired = fp32["launches"] < args.steps
     out = {
         "metric": METRIC,
         "value": fp32["mlups"],
@@ -884,8 +909,10 @@ def main():
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": fp32["achieved_gbs"] / HBM_PEAK_GBS,
-            "traffic": load_traffic(n),
-            "kernel": "xlbh::k_step<D3Q19, BGK, F32, float>",
+            "traffic": load_traffic(n, "step_pair" if paired else "step"),
+            "kernel": "xlbh::k_step_pair<D3Q19, BGK, F32, float>" if paired else "xlbh::k_step<D3Q19, BGK, F32, float>",
+            "launches": fp32["launches"],
+            "steps_per_launch": fp32["steps_per_launch"],
             "algorithmic_bytes_per_cell": fp32["bytes_per_lu"],
             "kernel_ms": fp32["kernel_ms"],
             "device_copy_gbs": copy["gbs"],
