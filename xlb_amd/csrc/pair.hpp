@@ -18,7 +18,9 @@
 // 160 KB of LDS, so one block of 16 waves runs per CU.  FP64 takes 7 rows (140 KB; a ninth wave
 // would cap the registers at 168 and spill).
 // Measured on the D3Q19 BGK step, 256^3 FP32: periodic 430 -> 282 us per step, cavity 434 -> 288
-// us, halfway walls 302 us; 512x256x256 860 -> 592 us; FP64 150x90x110 96 -> 65 us.
+// us, halfway walls 302 us; 512x256x256 860 -> 592 us; FP64 150x90x110 96 -> 65 us.  Bound by memory: a
+// pair on the 256^3 cavity reads and writes 2.84 GB (1.11 times its algorithmic bytes) in 564 us, 5.0
+// TB/s, the rate of a device copy; its VALU instructions take about half of that time.
 // What else was tried at 256^3 periodic (us per step): loads of the next plane before the first
 // update instead of after it 287 (and 320 on the cavity, whose boundary lookups then wait for
 // them); 14, 12 and 7 rows 302, 295 and 315 (the last with two blocks per CU); non-temporal loads
