@@ -66,3 +66,23 @@ def test_a_new_missing_mask_in_the_place_of_a_freed_one():
         assert torch.equal(st._bits.cpu(), bits), (i, again)
         del missing
     assert again  # it did happen here
+
+
+def test_a_stepper_with_state_can_be_copied_and_pickled():
+    """The copy derives its state from the masks it is given; results are the same."""
+    import copy
+    import pickle
+
+    BC = xa.operator.boundary_condition
+    policy = xa.PrecisionPolicy.FP32FP32
+    vs = xa.velocity_set.D2Q9(policy, xa.ComputeBackend.MI355X)
+    xa.init(velocity_set=vs, default_backend=xa.ComputeBackend.MI355X, default_precision_policy=policy)
+    grid = xa.grid.grid_factory((40, 24), compute_backend=xa.ComputeBackend.MI355X)
+    inner = grid.bounding_box_indices(remove_edges=True)
+    bcs = [BC.HalfwayBounceBackBC(indices=inner["bottom"]), BC.ExtrapolationOutflowBC(indices=inner["right"])]
+    st = xa.operator.stepper.IncompressibleNavierStokesStepper(grid, bcs)
+    f_0, f_1, bm, mm = st.prepare_fields()
+    f_0.mul_(1 + 0.02 * torch.rand(f_0.shape, generator=torch.Generator().manual_seed(1)).cuda())
+    want = st.run(f_0.clone(), f_1.clone(), bm, mm, 1.3, 7)[0]
+    for other in (copy.deepcopy(st), pickle.loads(pickle.dumps(st))):
+        assert torch.equal(other.run(f_0.clone(), f_1.clone(), bm, mm, 1.3, 7)[0], want)

@@ -13,7 +13,6 @@ table of prescribed values.  ``run`` moves the caller's step/swap loop below the
 """
 
 import ctypes
-import weakref
 
 import numpy as np
 import torch
@@ -101,7 +100,6 @@ class IncompressibleNavierStokesStepper(Stepper):
         self._far_patterns = None
         self._bc_cells = None
         self._mask_ref = None
-        self._missing_ref = None
 
     # ------------------------------------------------------------------ fields
     def prepare_fields(self, initializer=None):
@@ -174,8 +172,8 @@ class IncompressibleNavierStokesStepper(Stepper):
 
     def _sync_state(self, bc_mask, missing_mask):
         key = self._mask_key(bc_mask, missing_mask)
-        if key == self._state_key and self._missing_ref() is missing_mask:  # (ids are used again)
-            return
+        if key == self._state_key and packed_missing(missing_mask, self.lattice_id) is self._bits:
+            return  # (a new tensor may have the id, memory and version of a freed one, not its bits)
         _lib.require_cuda(bc_mask, missing_mask)
         ext = field_extents(bc_mask)
         expect_field(bc_mask, 1, ext, "bc_mask", torch.uint8)
@@ -205,7 +203,6 @@ class IncompressibleNavierStokesStepper(Stepper):
             for bc in aux_bcs:
                 bc.aux_data_init(None, None, bc_mask, missing_mask, aux=self._aux)
         self._mask_ref = bc_mask
-        self._missing_ref = weakref.ref(missing_mask)
         self._state_key = self._mask_key(bc_mask, missing_mask)
 
     def _far_outflow(self, bc_id, bc_mask):
